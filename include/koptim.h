@@ -197,6 +197,29 @@ int ko_qk_norm_rope_acc(float* acc, const void* q_w, const void* k_w, const void
  * out [M, I] = bf16(bf16(silu(gate)) * up). I % 8 == 0. */
 int ko_silu_mul(const void* gu, void* out, int M, int I, void* stream);
 
+/* ---- row kernels of the prompt forward ---------------------------------------
+ * The elementwise pieces of engine/engine.py:343-386 (the reference's
+ * engine/kernels/exact.py), with the bits of the torch operations that
+ * Transformers' Qwen3 modules run (the mean of squares added in torch's order).
+ *
+ * ko_prefill_norm: res <- bf16(res + delta) when delta is given; then
+ * out = bf16(w * bf16(res * rsqrt(mean(res^2) + eps))). Rows of n bf16 values,
+ * 256 <= n <= 8064, n % 4 == 0; every pointer 8-byte aligned.
+ * ko_prefill_qkv: the bf16 projections q [B*S, nq*d], k and v [B*S, nkv*d] of
+ * B prompts of S tokens at positions 0 .. S-1: q is normed and roped in place,
+ * k normed and roped into k_cache[b, h, s, :], v copied to v_cache[b, h, s, :]
+ * (strides in elements, sequence stride d = 128; cos/sin [max_pos, d], S <=
+ * max_pos; pointers 8-byte aligned, strides multiples of 4).
+ * ko_silu_mul2: out = bf16(bf16(silu(gate)) * up) over n values (n % 8 == 0,
+ * 16-byte aligned); out may be gate. */
+int ko_prefill_norm(void* res, const void* delta, const void* weight, void* out, int rows, int n,
+                    float eps, void* stream);
+int ko_prefill_qkv(void* q, const void* k, const void* v, const void* q_w, const void* k_w,
+                   const void* cos, const void* sin, void* k_cache, void* v_cache, int B, int S,
+                   long long cache_b_stride, long long cache_h_stride, float eps, int nq, int nkv,
+                   int d, int max_pos, void* stream);
+int ko_silu_mul2(const void* gate, const void* up, void* out, long long n, void* stream);
+
 /* ---- embedding gather + sum of squares ------------------------------------
  * Replaces engine/kernels/gemv.py:201-211 (_embed_ss_kernel) as launched by
  * embed_ss (gemv.py:214-216): h[m] = emb[ids[m]] ([V, H] bf16, ids int64),

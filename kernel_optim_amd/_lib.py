@@ -39,6 +39,11 @@ SIGNATURES = {
                             _c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _int, _ll, _ll,
                             _f, _int, _int, _int, _int, _c_void_p],
     "ko_silu_mul": [_c_void_p, _c_void_p, _int, _int, _c_void_p],
+    "ko_prefill_norm": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _int, _f, _c_void_p],
+    "ko_prefill_qkv": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+                       _c_void_p, _c_void_p, _c_void_p, _int, _int, _ll, _ll, _f, _int, _int,
+                       _int, _int, _c_void_p],
+    "ko_silu_mul2": [_c_void_p, _c_void_p, _c_void_p, _ll, _c_void_p],
     "ko_embed_ss": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _int, _int, _c_void_p],
     "ko_gemv": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                 _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _ll, _int, _int, _int, _int,

@@ -339,3 +339,56 @@ def silu_mul(gu, out):
     _check(gu, "gu", BF16, (M, 2 * I))
     _check(out, "out", BF16, (M, I))
     _lib.call("ko_silu_mul", _lib.ptr(gu), _lib.ptr(out), M, I, _lib.stream_ptr())
+
+
+# ---------------------------------------------------------------------------
+# Row kernels of the prompt forward (engine.py:343-386), with the bits of the torch
+# operations they replace.
+# ---------------------------------------------------------------------------
+def prefill_norm(res, delta, weight, out, eps):
+    """res <- res + delta (when given), out = Qwen3RMSNorm(res). res, delta and out are
+    bf16 of one shape with rows of 256 to 8064 values (a multiple of 4)."""
+    n = res.shape[-1]
+    _check(res, "res", BF16)
+    if delta is not None:
+        _check(delta, "delta", BF16, res.shape)
+    _check(weight, "weight", BF16, (n,))
+    _check(out, "out", BF16, res.shape)
+    _lib.call("ko_prefill_norm", _lib.ptr(res), _lib.ptr(delta), _lib.ptr(weight), _lib.ptr(out),
+              res.numel() // n, n, eps, _lib.stream_ptr())
+
+
+def prefill_qkv(q, k, v, q_w, k_w, cos, sin, k_cache, v_cache, eps):
+    """The prompt's projections q [.., nq*128], k and v [.., nkv*128] (B*S rows each,
+    positions 0..S-1): per-head RMSNorm + RoPE of q in place and of k into the cache's
+    first S slots, v copied there. k_cache/v_cache: one layer, [B, nkv, cap, 128]."""
+    B, nkv, cap, d = k_cache.shape
+    M = q.numel() // q.shape[-1]
+    _need(M % B == 0, "rows must be B*S")
+    _check(q, "q", BF16)
+    _check(k, "k", BF16)
+    _check(v, "v", BF16)
+    _need(q.shape[-1] % d == 0 and k.shape[-1] == nkv * d and tuple(k.shape) == tuple(v.shape)
+          and k.numel() == M * nkv * d, "q, k and v must be [B*S, heads*d]")
+    _check(q_w, "q_w", BF16, (d,))
+    _check(k_w, "k_w", BF16, (d,))
+    _check(cos, "cos", BF16)
+    _check(sin, "sin", BF16)
+    _need(cos.dim() == 2 and sin.dim() == 2 and cos.shape[1] == d and sin.shape[1] == d,
+          "cos/sin must be [rows, d]")
+    _check_cache(k_cache, "k_cache", B, nkv, cap, d)
+    _check_cache(v_cache, "v_cache", B, nkv, cap, d)
+    _need(k_cache.stride() == v_cache.stride(), "k_cache and v_cache must share strides")
+    _lib.call("ko_prefill_qkv", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(q_w),
+              _lib.ptr(k_w), _lib.ptr(cos), _lib.ptr(sin), _lib.ptr(k_cache), _lib.ptr(v_cache),
+              B, M // B, k_cache.stride(0), k_cache.stride(1), eps, q.shape[-1] // d, nkv, d,
+              min(cap, cos.shape[0], sin.shape[0]), _lib.stream_ptr())
+
+
+def silu_mul2(gate, up, out):
+    """out = bf16(bf16(silu(gate)) * up) over tensors of one shape; out may be gate."""
+    _check(gate, "gate", BF16)
+    _check(up, "up", BF16, gate.shape)
+    _check(out, "out", BF16, gate.shape)
+    _lib.call("ko_silu_mul2", _lib.ptr(gate), _lib.ptr(up), _lib.ptr(out), gate.numel(),
+              _lib.stream_ptr())

@@ -141,3 +141,17 @@ def test_gemv_host_path_of_every_layout_without_gpu(libpath):
     # ARGMAX partials: 160 tiles on 160 workgroups, 16 or 32 rows each
     assert h.ko_gemv_argmax_scratch(2560, 2, 1, 0) == 2 * 16 * 160
     assert h.ko_gemv_argmax_scratch(2560, 2, 1, 2) == 2 * 32 * 160
+
+
+def test_prefill_row_kernels_refuse_bad_shapes_without_gpu(libpath):
+    from kernel_optim_amd import _lib
+    h = _lib.lib()
+    P = 1 << 20
+    for n, st in [(252, -95), (8068, -95), (2558, -95)]:
+        assert h.ko_prefill_norm(P, None, P, P, 8, n, 1e-6, None) == st
+    assert h.ko_prefill_norm(P, P + 4, P, P, 8, 2560, 1e-6, None) == -22
+    args = [P] * 9
+    assert h.ko_prefill_qkv(*args, 1, 9, 1024, 1024, 1e-6, 32, 8, 128, 8, None) == -22
+    assert h.ko_prefill_qkv(*args, 1, 8, 1024, 1024, 1e-6, 32, 8, 64, 8, None) == -95
+    assert h.ko_prefill_qkv(*args, 1, 8, 1024, 1022, 1e-6, 32, 8, 128, 8, None) == -22
+    assert h.ko_silu_mul2(P, P, P, 12, None) == -22
