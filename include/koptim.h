@@ -278,11 +278,32 @@ int ko_embed_ss(const long long* ids, const void* emb, void* h, float* ss, int M
  *           weights; a slice runs on the fewest tiles that hold it). part is its
  *           scratch (part_len >= ko_gemv_argmax_scratch(N, 4, 10, waves)), with
  *           the rules of layout 3's.
+ * layout 5: MFMA tiles on the tiled weight copy, M <= 64 per launch slice, `rows`
+ *           column tiles per workgroup, K in `waves` slices. Behind a norm (norm
+ *           != 0, K = 2560, `waves` 1): F32 or BF16 with `rows` 2, SWIGLU 3,
+ *           ARGMAX 4 or 6; x is normalised by a launch of its own. RESID without
+ *           a norm (N % 4 == 0, N <= 8192): `rows` 3 in 4 slices (K = 4096,
+ *           9728) or 5 in 8 (K = 9728); a second launch adds the slices' fp32
+ *           sums in slice order (deterministic) and the residual. part is its
+ *           scratch (part_len >= ko_gemv_argmax_scratch(N, 5, rows, waves));
+ *           calls that share it must not overlap.
  * K % 8 == 0. M larger than a slice is processed in several launches. */
 int ko_gemv(const void* x, const void* w, void* y, const void* nw, const float* ss, void* h,
             float* ss_out, long long* ids, int* pos_inc, const void* next_emb, void* next_h,
             float* part, long long part_len, int M, int N, int K, int epi, int norm,
             int accumulate, int layout, int rows, int waves, float eps, void* stream);
+
+/* ko_gemv with layout 5 (up to 64 rows, no ARGMAX) tied to its neighbours. next_xn
+ * (RESID, N % 32 == 0): also receives bf16(next_nw * bf16(h * rstd)) of the new h, the
+ * NORM prologue of the projection that reads h next, in that projection's operand order:
+ * for k step k / 32 and row tile m / 16 of ceil(M / 16) a block of 512 elements, element
+ * (m, k) at ((m % 16) + 16 (k % 32 / 8)) * 8 + k % 8 (64 * N elements; rows past M are
+ * not written). xn (norm projections): the input in that form, read in place of x.
+ * Either may be NULL. The bits are those of ko_gemv's own norm of h. */
+int ko_gemv_chained(const void* x, const void* w, void* y, const void* nw, const float* ss,
+                    void* h, float* ss_out, const void* xn, const void* next_nw, void* next_xn,
+                    float* part, long long part_len, int M, int N, int K, int epi, int norm,
+                    int rows, int waves, float eps, void* stream);
 
 /* The decode step's tail in one call: the LM head GEMV with the greedy argmax
  * (ko_gemv with epi 4, ARGMAX, and a NORM prologue when nw != NULL), followed
@@ -312,8 +333,8 @@ int ko_lm_head_argmax(const void* x, const void* w, const void* nw, const float*
                       int waves, float eps, void* stream);
 
 /* Number of fp32 scratch elements ko_gemv needs for N columns with this launch
- * configuration: the ARGMAX partials (epi 4) of layouts 0-2, or layout 3's
- * (rows > 1) and layout 4's slots and counters. A size, not a status; -1 for
+ * configuration: the ARGMAX partials (epi 4) of layouts 0-2, layout 3's
+ * (rows > 1) and layout 4's slots and counters, or layout 5's sums and inputs. A size, not a status; -1 for
  * bad arguments.
  * Helper of ko_gemv, no reference counterpart. */
 long long ko_gemv_argmax_scratch(int N, int layout, int rows, int waves);

@@ -48,6 +48,9 @@ SIGNATURES = {
     "ko_gemv": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                 _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _ll, _int, _int, _int, _int,
                 _int, _int, _int, _int, _int, _f, _c_void_p],
+    "ko_gemv_chained": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+                        _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _ll, _int, _int,
+                        _int, _int, _int, _int, _int, _f, _c_void_p],
     "ko_lm_head_argmax": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                           _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _int,
                           _c_void_p, _c_void_p, _int, _c_void_p, _c_void_p, _c_void_p, _ll, _int,

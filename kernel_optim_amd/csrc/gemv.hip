@@ -271,6 +271,7 @@ bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 long long parts_for(int N, int layout, int rows, int waves) {
   if (layout == 0) return (N + rows - 1) / rows;
   if (layout == 2) return mfma_grid(N, rows);
+  if (layout == 5) return rows_parts(N, rows);
   if (layout != 1 || waves < 1) return 0;  // layouts 3 and 4 have no ARGMAX partials
   const long long units = (N + rows - 1) / rows;
   return ((units + waves - 1) / waves) * waves;
@@ -280,7 +281,7 @@ int gemv_impl(const void* x, const void* w, void* y, const void* nw, const float
               float* ss_out, long long* ids, int* pos_inc, const void* next_emb, void* next_h,
               float* part, long long part_len, int M, int N, int K, int epi, int norm,
               int accumulate, int layout, int rows, int waves, float eps, const StepTail& tail,
-              hipStream_t s) {
+              const RowsChain& chain, hipStream_t s) {
   if (!x || !w || M < 1 || N < 1 || K < 8 || (K & 7)) return KO_EINVAL;
   if (epi < EPI_F32 || epi > EPI_ARGMAX) return KO_EINVAL;
   if (!al16(x) || !al16(w)) return KO_EINVAL;
@@ -307,8 +308,18 @@ int gemv_impl(const void* x, const void* w, void* y, const void* nw, const float
       return KO_ENOTSUP;
     if (waves != 0 && waves != 2 && waves != 4) return KO_ENOTSUP;  // row tiles: 0 (one), 2, 4
     if (!part || !al16(part) || part_len < sk_scratch(N, waves ? waves : 1)) return KO_ERANGE;
+  } else if (layout == 5) {
+    if (!rows_supported(N, K, epi, norm != 0, rows, waves)) return KO_ENOTSUP;
+    if (!part || !al16(part) || part_len < rows_scratch(N, rows, waves)) return KO_ERANGE;
   } else {
     return KO_EINVAL;
+  }
+  if (chain.xn || chain.next_xn) {  // one weight pass: the chained rows are one operand
+    if (layout != 5 || M > ROWS_MAX) return KO_ENOTSUP;
+    if (chain.xn && (epi == EPI_RESID || !al16(chain.xn))) return KO_EINVAL;
+    if (chain.next_xn && (epi != EPI_RESID || !al16(chain.next_xn) || !chain.next_nw ||
+                          !al16(chain.next_nw) || N % 32))
+      return KO_EINVAL;
   }
   const int mstep = mstep_for(layout, waves);
   const long long nparts = parts_for(N, layout, rows, waves);
@@ -332,7 +343,7 @@ int gemv_impl(const void* x, const void* w, void* y, const void* nw, const float
     a.ss = ss ? ss + m0 : nullptr;
     a.h = h ? static_cast<uint16_t*>(h) + (long long)m0 * N : nullptr;
     a.ss_out = ss_out ? ss_out + m0 : nullptr;
-    a.part = reinterpret_cast<float2*>(part);
+    a.part = reinterpret_cast<float2*>(layout == 5 && waves == 1 ? part + ROWS_XN : part);
     a.nparts = (int)nparts;
     a.mrows = mr;
     a.N = N;
@@ -349,6 +360,8 @@ int gemv_impl(const void* x, const void* w, void* y, const void* nw, const float
     else if (layout == 3)
       st = launch_layout3(a, epi, norm != 0, rows, reinterpret_cast<int*>(part),
                           part + ((N + 15) / 16 + 63) / 64 * 64, s);
+    else if (layout == 5)
+      st = launch_layout5(a, epi, norm != 0, rows, waves, chain, part, s);
     else
       st = launch_layout4(a, epi, sk_tiles(waves, mr), reinterpret_cast<int*>(part),
                           part + ((N + 15) / 16 + 63) / 64 * 64, s);
@@ -382,7 +395,20 @@ int ko_gemv(const void* x, const void* w, void* y, const void* nw, const float* 
             int accumulate, int layout, int rows, int waves, float eps, void* stream) {
   const StepTail none = {};
   return gemv_impl(x, w, y, nw, ss, h, ss_out, ids, pos_inc, next_emb, next_h, part, part_len, M,
-                   N, K, epi, norm, accumulate, layout, rows, waves, eps, none,
+                   N, K, epi, norm, accumulate, layout, rows, waves, eps, none, RowsChain{},
+                   static_cast<hipStream_t>(stream));
+}
+
+int ko_gemv_chained(const void* x, const void* w, void* y, const void* nw, const float* ss,
+                    void* h, float* ss_out, const void* xn, const void* next_nw, void* next_xn,
+                    float* part, long long part_len, int M, int N, int K, int epi, int norm,
+                    int rows, int waves, float eps, void* stream) {
+  const StepTail none = {};
+  const RowsChain chain = {static_cast<const uint16_t*>(xn), static_cast<const uint16_t*>(next_nw),
+                           static_cast<uint16_t*>(next_xn)};
+  if (epi == EPI_ARGMAX) return KO_ENOTSUP;
+  return gemv_impl(x, w, y, nw, ss, h, ss_out, nullptr, nullptr, nullptr, nullptr, part, part_len,
+                   M, N, K, epi, norm, 0, 5, rows, waves, eps, none, chain,
                    static_cast<hipStream_t>(stream));
 }
 
@@ -412,7 +438,7 @@ int ko_lm_head_argmax(const void* x, const void* w, const void* nw, const float*
   }
   return gemv_impl(x, w, logits, nw, ss, nullptr, nullptr, ids, pos, next_emb, next_h, part,
                    part_len, M, N, K, EPI_ARGMAX, nw != nullptr, 0, layout, rows, waves, eps,
-                   tail, static_cast<hipStream_t>(stream));
+                   tail, RowsChain{}, static_cast<hipStream_t>(stream));
 }
 
 int ko_gemv_tile(const void* w, void* wt, int rows, int K, void* stream) {
@@ -437,7 +463,8 @@ int ko_argmax_rows(const void* x, long long ld, int M, int N, long long* ids, vo
 // fp32 scratch elements ko_gemv needs for EPI 4 (ARGMAX) with this layout
 // (a size, not a status; -1 for bad arguments).
 long long ko_gemv_argmax_scratch(int N, int layout, int rows, int waves) {
-  if (N < 1 || rows < 1 || (layout == 1 && waves < 1) || layout < 0 || layout > 4) return -1;
+  if (N < 1 || rows < 1 || (layout == 1 && waves < 1) || layout < 0 || layout > 5) return -1;
+  if (layout == 5) return waves < 1 ? -1 : rows_scratch(N, rows, waves);
   if (layout == 3) return rows > 1 ? ks_scratch(N, rows) : 0;
   if (layout == 4) return sk_scratch(N, waves == 2 || waves == 4 ? waves : 1);
   return 2LL * mstep_for(layout, waves) * parts_for(N, layout, rows, waves);

@@ -1,6 +1,6 @@
-// Launchers of the five GEMV layouts, compiled in their own sources
+// Launchers of the GEMV layouts, compiled in their own sources
 // (gemv_block.hip: layout 0; gemv_wave.hip: layout 1; gemv_mfma.hip: layouts 2,
-// 3 and 4) and called
+// 3 and 4; gemm_rows.hip: layout 5) and called
 // by the C entry points in gemv.hip, plus the shape rules those entry points
 // validate against.
 #pragma once
@@ -30,6 +30,38 @@ int launch_layout3(const GemvArgs& a, int epi, bool norm, int slices, int* ctr, 
 // layout 4: stream-K over the tiles' K chunks; mt row tiles of 16 rows of x per weight pass
 int launch_layout4(const GemvArgs& a, int epi, int mt, int* ctr, float* slots, hipStream_t s);
 
+// layout 5: `tn` column tiles per workgroup, K in `slices`; up to ROWS_MAX rows per
+// weight pass. What ties projections together: x already normalised (operand order),
+// and for RESID the next projection's norm gain and normalised input.
+constexpr int ROWS_MAX = 64;
+struct RowsChain {
+  const uint16_t* xn;
+  const uint16_t* next_nw;
+  uint16_t* next_xn;
+};
+int launch_layout5(GemvArgs a, int epi, bool norm, int tn, int slices, const RowsChain& chain,
+                   float* part, hipStream_t s);
+// K = 2560 behind a norm (F32 and BF16 with 2 tiles per workgroup, SWIGLU 3, ARGMAX 4 or
+// 6), one slice; RESID without a norm, 4 slices of 3 tiles (K = 4096, 9728) or 8 of 5
+// (9728): about one workgroup per CU at N = 2560.
+inline bool rows_supported(int N, int K, int epi, bool norm, int tn, int slices) {
+  if (epi == EPI_RESID)
+    return !norm && (N & 3) == 0 && N <= 8192 &&
+           ((slices == 4 && tn == 3 && (K == 4096 || K == 9728)) ||
+            (slices == 8 && tn == 5 && K == 9728));
+  if (!norm || K != 2560 || slices != 1) return false;
+  if (epi == EPI_ARGMAX) return tn == 4 || tn == 6;
+  return tn == (epi == EPI_SWIGLU ? 3 : 2);
+}
+// Scratch (fp32 elements): the slices' sums, or with one slice the normalised x and the
+// ARGMAX partials behind it.
+constexpr long long ROWS_XN = ROWS_MAX * 2560 / 2;
+inline long long rows_parts(int N, int tn) { return ((N + 15) / 16 + tn - 1) / tn; }
+inline long long rows_scratch(int N, int tn, int slices) {
+  if (slices > 1) return (long long)slices * ROWS_MAX * N;
+  return ROWS_XN + 2LL * ROWS_MAX * rows_parts(N, tn);
+}
+
 // Workgroups of the layout-2 grid: at most MFMA_CUS * per_cu, and of those the
 // fewest that keep the most tiles per workgroup at its minimum, so every
 // workgroup runs the same number of tiles (but the last ones, one fewer). A
@@ -54,11 +86,12 @@ inline bool mfma_supported(int K, int epi, int mt = 1) {
 }
 
 // Rows of x per launch of a layout: 4 (layout 1), 32 (layouts 2 and 4 with two
-// row tiles, waves == 2), 64 (layout 4 with four, waves == 4), else 16.
+// row tiles, waves == 2), 64 (layout 4 with four, waves == 4; layout 5), else 16.
 inline int mstep_for(int layout, int waves) {
   if (layout == 1) return 4;
   if ((layout == 2 || layout == 4) && waves == 2) return 32;
   if (layout == 4 && waves == 4) return 64;
+  if (layout == 5) return ROWS_MAX;
   return 16;
 }
 // Row tiles of a launch slice of mr rows under a layout-4 `waves` (0, 2 or 4):

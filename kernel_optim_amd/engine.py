@@ -43,7 +43,7 @@ import time
 import torch
 
 from .kernels.fused import DecodeAttention, add_rms_norm, qk_norm_rope, rope_rows, silu_mul
-from .kernels.gemv import (EPI_ARGMAX, EPI_BF16, EPI_RESID, EPI_SWIGLU, Gemv, argmax_rows,
+from .kernels.gemv import (EPI_ARGMAX, EPI_BF16, EPI_RESID, EPI_SWIGLU, ROWS_MAX, Gemv, argmax_rows,
                            embed_ss, tile_weights, uses_tiled)
 from .model import Qwen3Config, load_checkpoint, random_weights
 from .prefill import prefill
@@ -68,9 +68,9 @@ ATTN_SPLIT = int(os.environ.get("ENGINE_ATTN_SPLIT", "-1"))
 # keeps the faster, as the reference does (engine.py:197-208); "fused" or
 # "hipblaslt" takes one
 DECODE_GRAPH = os.environ.get("ENGINE_DECODE_GRAPH", "auto")
-# The fused GEMVs read each weight once for up to 32 rows (B = 32: 8,619 tok/s
-# against 7,544 on hipBLASLt); at 33..64 rows qkv, gate/up and the LM head take
-# two weight passes (B = 64: 9,538 against 11,599 tok/s on hipBLASLt).
+# The fused GEMVs of any width read each weight once for up to 32 rows (B = 32: 8,619
+# tok/s against 7,544 on hipBLASLt); at 33..64 rows only layout 5 does, so "auto" takes
+# the fused step there for the widths that it serves (rows_served).
 FUSED_MAX_B = 32
 FUSED_MAX_TIMED = 64  # "timed": both graphs up to here (engine.py:44)
 # verify-step attention: the K+1 tokens of a sequence as rows of the one-token
@@ -178,7 +178,18 @@ def attn_units_per_seq(B, nkv):
     return max(1, 256 // (B * nkv)) if 3 <= B <= 64 else 0
 
 
-def build_decode_gemvs(cfg, M, raw, deadline, tiled_fn=None, tune=True, log=""):
+def rows_served(cfg):
+    """Whether GEMV layout 5 (up to 64 rows per weight pass) serves all the projections of
+    this model's decode step."""
+    H, e = cfg.hidden, cfg.eps
+    return all(g.rows_cfgs() for g in (
+        Gemv(64, cfg.nqkv, H, EPI_BF16, norm=True, eps=e),
+        Gemv(64, H, cfg.nq * cfg.head_dim, EPI_RESID, norm=False, eps=e),
+        Gemv(64, cfg.inter, H, EPI_SWIGLU, norm=True, eps=e),
+        Gemv(64, H, cfg.inter, EPI_RESID, norm=False, eps=e)))
+
+
+def build_decode_gemvs(cfg, M, raw, deadline, tiled_fn=None, tune=True, log="", chain=False):
     """The decode step's five fused projections for M rows (the reference's
     _setup_fused set, engine.py:256-262, with the LM head's greedy selection
     fused in): qkv (RMSNorm prologue, bf16 out), o (+ residual), gate/up (RMSNorm
@@ -186,7 +197,9 @@ def build_decode_gemvs(cfg, M, raw, deadline, tiled_fn=None, tune=True, log=""):
     ``raw`` maps each name to its per-layer row-major weights; with ``tune`` each
     Gemv is timed over them (Gemv.tune). ``tiled_fn(name, weights)`` returns the
     MFMA-tiled copies for a projection that has tiled candidates (None: tune
-    makes them). Returns (gemvs, weights in each one's launch layout)."""
+    makes them). ``chain``: the caller passes decode_layer the next layer's norm, so
+    qkv's input comes normalised from the layer before. Returns (gemvs, weights in each
+    one's launch layout)."""
     H, e = cfg.hidden, cfg.eps
     gv = dict(
         qkv=Gemv(M, cfg.nqkv, H, EPI_BF16, norm=True, eps=e),
@@ -196,39 +209,70 @@ def build_decode_gemvs(cfg, M, raw, deadline, tiled_fn=None, tune=True, log=""):
         lm=Gemv(M, cfg.vocab, H, EPI_ARGMAX, norm=True, eps=e),
     )
     W = {}
-    for name, g in gv.items():
+    for name in ("o", "gu", "down", "qkv", "lm"):   # a producer before its consumer
         if name not in raw:
             continue
+        g = gv[name]
         tiled = None
         if any(uses_tiled(c) for c in g.candidates()):
             tiled = (tiled_fn(name, raw[name]) if tiled_fn is not None
                      else [tile_weights(w, swiglu=name == "gu") for w in raw[name]])
-        if tune:
-            g.tune(raw[name], deadline, tiled=tiled)
+        if tune and M > 16 and g.rows_cfgs():
+            # From 17 rows on the better layout is clear: layout 5 for the layers, where o and
+            # gate/up gain more as a pair (one norm less) than the tuner sees (32 rows: 9.7 +
+            # 20.5 us against 10.5 + 24.3, down 15.1 against 19.5, qkv with its norm 12.0
+            # against 14.3), down in 8 slices above 32 rows (64 rows 19.2 against 20.0, 32
+            # rows 15.6 against 15.1); the LM head on layout 2 up to 32 rows (150 against 158
+            # us; 48 rows 285 against 191).
+            g.cfg = g.rows_cfgs()[0 if M > 32 else -1]
+            if name == "lm" and M <= 32:
+                g.cfg = (2, 1, 2)
+            _log(f"{log}gemv {name} M={M} cfg={g.cfg} (rule)")
+        elif tune:
+            given = (name == "gu" and gv["o"].cfg[0] == 5 or
+                     name == "qkv" and chain and gv["down"].cfg[0] == 5)
+            g.tune(raw[name], deadline, tiled=tiled, given=given)
             _log(f"{log}gemv {name} M={M} cfg={g.cfg} {g.us:.1f}us candidates={g.tune_log}")
         W[name] = tiled if uses_tiled(g.cfg) else raw[name]
     return gv, W
 
 
+def _chain(gv, src, dst, gain):
+    """What ties residual projection ``src`` to norm projection ``dst`` (Gemv.__call__'s
+    nxt and xn), where both run on layout 5 in one weight pass; else (None, None)."""
+    s, d = gv[src], gv[dst]
+    if gain is None or s.cfg[0] != 5 or d.cfg[0] != 5 or s.M > ROWS_MAX or s.N != d.K:
+        return None, None
+    buf = d.xn_buffer(gain.device)
+    return (gain, buf), buf
+
+
 def decode_layer(gv, W, i, lw, attn, h, qkv, attn_out, act, k_cache, v_cache, cos, sin, pos,
-                 rope, eps, fuse_o):
+                 rope, eps, fuse_o, next_norm=None, normed=False):
     """Layer i of the one-token decode step (engine.py:278-287 in this package's
     launches): qkv GEMV (RMSNorm prologue) -> attention (q/k norm + RoPE + KV
     append at pos, split-K partials, last-unit merge), with the o projection and
     its residual add in the same launch when ``fuse_o`` -> o GEMV (+ residual)
     otherwise -> gate/up GEMV (RMSNorm prologue, SwiGLU) -> down GEMV (+ residual).
     h [B, H] is the residual stream, updated in place; k_cache/v_cache are the
-    layer's [B, nkv, cap, d] slices; rope the step's RoPE rows (rope_rows)."""
-    gv["qkv"](h, W["qkv"][i], y=qkv, nw=lw["w_in"])
+    layer's [B, nkv, cap, d] slices; rope the step's RoPE rows (rope_rows). On GEMV layout 5
+    the residual projections leave the normalised input of the projection after them:
+    o that of gate/up, and down, given ``next_norm`` (the next layer's input norm gain),
+    that of the next call's qkv, which takes it with ``normed`` (nothing may change h in
+    between)."""
+    xn = _chain(gv, "down", "qkv", lw["w_in"])[1] if normed else None
+    gv["qkv"](h, W["qkv"][i], y=qkv, nw=lw["w_in"], xn=xn)
+    xn = None
     if fuse_o:
         attn.decode_qkv_oproj(qkv, lw["q_norm"], lw["k_norm"], cos, sin, pos, k_cache, v_cache,
                               attn_out, eps, lw["o"], h, rope=rope)
     else:
         attn.decode_qkv(qkv, lw["q_norm"], lw["k_norm"], cos, sin, pos, k_cache, v_cache,
                         attn_out, eps, rope=rope)
-        gv["o"](attn_out, W["o"][i], h=h)
-    gv["gu"](h, W["gu"][i], y=act, nw=lw["w_post"])
-    gv["down"](act, W["down"][i], h=h)
+        nxt, xn = _chain(gv, "o", "gu", lw["w_post"])
+        gv["o"](attn_out, W["o"][i], h=h, nxt=nxt)
+    gv["gu"](h, W["gu"][i], y=act, nw=lw["w_post"], xn=xn)
+    gv["down"](act, W["down"][i], h=h, nxt=_chain(gv, "down", "qkv", next_norm)[0])
 
 
 class Engine:
@@ -341,7 +385,8 @@ class Engine:
         deadline = time.monotonic() + TUNE_BUDGET_S
         kind = self.decode_graph
         if kind == "auto":
-            kind = "fused" if B <= FUSED_MAX_B else "hipblaslt"
+            kind = ("fused" if B <= (ROWS_MAX if rows_served(cfg) else FUSED_MAX_B)
+                    else "hipblaslt")
         elif kind == "timed" and B > FUSED_MAX_TIMED:
             kind = "hipblaslt"
         self.step_times = {}
@@ -368,7 +413,7 @@ class Engine:
         """The fused-GEMV decode step: tuned GEMVs (with MFMA weight copies where
         the tuner takes them) and its captured graph."""
         self.gv, self.gw = build_decode_gemvs(self.cfg, self.B, raw, deadline, self._tiled,
-                                              tune=TUNE)
+                                              tune=TUNE, chain=True)
         return self._capture(self._step1)
 
     def _setup_mm(self):
@@ -470,10 +515,12 @@ class Engine:
         # previous step's LM head tail (or by the prefill hand-off)
         h = self.h
         fuse_o = FUSE_OPROJ and self.attn.oproj_fusable()
-        for i, lw in enumerate(self.w["layers"]):
+        L = self.w["layers"]
+        for i, lw in enumerate(L):
             decode_layer(g, W, i, lw, self.attn, h, self.qkv, self.attn_out, self.act,
                          self.k_cache[i], self.v_cache[i], self._cos, self._sin, self.pos,
-                         self.rope, cfg.eps, fuse_o)
+                         self.rope, cfg.eps, fuse_o,
+                         next_norm=L[i + 1]["w_in"] if i + 1 < len(L) else None, normed=i > 0)
         # LM head + greedy ids + pos += 1 + the next step's embedding rows and RoPE
         # rows + the ids into the pinned host ring, in one call
         g["lm"](h, W["lm"][0], y=self.logits, nw=self.w["final_norm"], ids=self.ids,

@@ -25,7 +25,10 @@ each weight load; layout 4 with ``waves`` = 4: 64 rows) and read a tiled copy of
 the K range of a tile cut into ``rows`` slices merged by the tile's last slice,
 layout 4 with each tile cut into 16 K chunks dealt out 10 per workgroup and
 merged by the tile's last workgroup (no atomics on the output in either, so the
-F32 epilogue is a plain store).
+F32 epilogue is a plain store). Layout 5 (``(5, tiles, slices)``) takes up to 64 rows
+per weight pass: a norm projection's x is normalised by a launch of its own, or by
+the residual projection before it (``nxt`` / ``xn`` of ``__call__``), and a residual
+projection's K slices are added by one more launch.
 ``allow_split`` is accepted for signature compatibility.
 
 Drop-in rule for the tiled layouts: the default configuration (``cfg`` before
@@ -45,11 +48,12 @@ from .. import _lib
 from .fused import BF16, _cdiv, _check, _need
 
 EPI_F32, EPI_BF16, EPI_RESID, EPI_SWIGLU, EPI_ARGMAX = 0, 1, 2, 3, 4
+ROWS_MAX = 64   # rows per weight pass of layout 5
 
 
 def uses_tiled(cfg):
-    """Layouts 2, 3 and 4 (MFMA) read the tile_weights copy of the weights."""
-    return cfg[0] in (2, 3, 4)
+    """Layouts 2 to 5 (MFMA) read the tile_weights copy of the weights."""
+    return cfg[0] in (2, 3, 4, 5)
 
 
 def is_tiled(w):
@@ -68,6 +72,7 @@ class Gemv:
         self.allow_split = allow_split
         self.cfg = self.candidates()[0]
         self._part = None
+        self._rows = self._xn = None
         self._tiles = {}   # id(row-major weight) -> (weakref to it, its tiled copy)
         self.us = float("nan")
         self.tune_log = []
@@ -102,6 +107,25 @@ class Gemv:
         return (not self.norm and self.epi in (EPI_F32, EPI_BF16, EPI_RESID)
                 and self.K % 512 == 0 and self.K // 512 in (19, 8, 5))
 
+    def rows_cfgs(self):
+        """Layout 5's configurations of this projection, the better one at more than 32
+        rows first (gemv_launch.h, rows_supported)."""
+        if self.epi == EPI_RESID:
+            if self.norm or self.N % 4 or self.N > 8192:
+                return []
+            return {4096: [(5, 3, 4)], 9728: [(5, 5, 8), (5, 3, 4)]}.get(self.K, [])
+        if not self.norm or self.K != 2560:
+            return []
+        return {EPI_SWIGLU: [(5, 3, 1)], EPI_ARGMAX: [(5, 6, 1), (5, 4, 1)]}.get(
+            self.epi, [(5, 2, 1)])
+
+    def xn_buffer(self, device):
+        """The normalised input of a layout-5 norm projection, which the residual
+        projection before it fills (``nxt``): one weight pass of 64 rows."""
+        if self._xn is None or self._xn.device != device:
+            self._xn = torch.zeros(ROWS_MAX * self.K, dtype=BF16, device=device)
+        return self._xn
+
     def candidates(self):
         """Launch configurations, the default first. The default is always a
         row-major layout, so an untuned Gemv runs on the weights the caller holds.
@@ -112,7 +136,8 @@ class Gemv:
         per workgroup at its minimum; ``(2, per_cu, 2)``: 32 rows per weight
         pass, offered above 16 rows), layout 3 splits its tiles' K range and
         layout 4 (``(4, 10, 0)``; ``(4, 10, 2)`` / ``(4, 10, 4)`` with 32 / 64
-        rows) deals the tiles' 16 K chunks out 10 per workgroup."""
+        rows) deals the tiles' 16 K chunks out 10 per workgroup, layout 5 (rows_cfgs)
+        takes up to 64 rows per weight pass."""
         out = []
         mfma = [(2, 2, 0), (2, 1, 0)] if self.M >= 2 and self.mfma_ok() else []
         mfma += [(2, 2, 2), (2, 1, 2)] if self.M > 16 and self.mfma2_ok() else []
@@ -120,6 +145,7 @@ class Gemv:
         mfma += [(4, 10, 0)] if self.M >= 2 and self.sk_ok() else []
         mfma += [(4, 10, 2)] if self.M > 16 and self.sk_ok() else []
         mfma += [(4, 10, 4)] if self.M > 32 and self.sk_ok() else []
+        mfma += self.rows_cfgs() if self.M >= 2 else []
         if self.M <= 4 and (not self.norm or self.M * self.K * 2 <= 40960):
             per_wave = (4, 2, 1) if self.N >= 32768 else (1, 2, 4)
             for rows in per_wave:
@@ -133,11 +159,15 @@ class Gemv:
     def _scratch(self, device, cfg):
         """fp32 scratch of the ARGMAX partials or of layout 3's and 4's slots and
         arrival counters (allocated zeroed: the counters start at zero and every
-        launch leaves them there)."""
+        launch leaves them there); layout 5 has one of its own, as it leaves sums
+        where those counters are."""
         n = _lib.lib().ko_gemv_argmax_scratch(self.N, *cfg)
-        if self._part is None or self._part.device != device or self._part.numel() < n:
-            self._part = torch.zeros(max(n, 2), dtype=torch.float32, device=device)
-        return self._part
+        name = "_rows" if cfg[0] == 5 else "_part"
+        t = getattr(self, name)
+        if t is None or t.device != device or t.numel() < n:
+            t = torch.zeros(max(n, 2), dtype=torch.float32, device=device)
+            setattr(self, name, t)
+        return t
 
     def _weight_for(self, w, cfg):
         """The weight tensor this configuration reads: ``w`` itself, or for a tiled
@@ -159,8 +189,11 @@ class Gemv:
                 self._tiles[id(w)] = (weakref.ref(w), t)
 
     def __call__(self, x, w, y=None, nw=None, ss=None, h=None, ss_out=None, cfg=None, ids=None,
-                 pos_inc=None, next_emb=None, next_h=None, rope=None, ring=None):
-        """ARGMAX extras: ``pos_inc`` ([M] int32) is advanced by one; with
+                 pos_inc=None, next_emb=None, next_h=None, rope=None, ring=None, xn=None, nxt=None):
+        """Layout 5, up to 64 rows: a residual projection with ``nxt = (gain, buffer)`` also
+        leaves the RMSNorm of its new h with that gain in the buffer (``xn_buffer`` of the
+        projection that reads h next), and a norm projection with ``xn`` (that buffer)
+        reads it in place of x. ARGMAX extras: ``pos_inc`` ([M] int32) is advanced by one; with
         ``next_emb`` ([N, K] bf16, the embedding) the chosen ids' rows are gathered
         into ``next_h`` ([M, K] bf16), the next decode step's input. The decode
         step's tail (ko_lm_head_argmax): ``rope = (cos, sin, out)`` writes the
@@ -216,7 +249,24 @@ class Gemv:
                 if len(ring) == 3 and ring[2] is not None:
                     _check(ring[2], "ring err", torch.int32, (1,))
         part = (self._scratch(x.device, (layout, rows, waves))
-                if epi == EPI_ARGMAX or (layout == 3 and rows > 1) or layout == 4 else None)
+                if epi == EPI_ARGMAX or (layout == 3 and rows > 1) or layout in (4, 5) else None)
+        if xn is not None or nxt is not None:
+            _need(layout == 5 and M <= ROWS_MAX and epi != EPI_ARGMAX,
+                  "xn and nxt serve layout 5, up to 64 rows, without ARGMAX")
+            gain, buf = nxt if nxt is not None else (None, None)
+            if buf is not None:
+                _need(epi == EPI_RESID, "nxt serves a residual projection")
+                _check(gain, "next gain", BF16, (N,))
+                _check(buf, "next input", BF16, (ROWS_MAX * N,))
+            if xn is not None:
+                _need(self.norm, "xn serves a norm projection")
+                _check(xn, "xn", BF16, (ROWS_MAX * K,))
+            _lib.call("ko_gemv_chained", _lib.ptr(x), _lib.ptr(w), _lib.ptr(y),
+                      _lib.ptr(nw) if self.norm else None, _lib.ptr(ss) if self.norm else None,
+                      _lib.ptr(h), _lib.ptr(ss_out), _lib.ptr(xn), _lib.ptr(gain), _lib.ptr(buf),
+                      _lib.ptr(part), part.numel(), M, N, K, epi, int(self.norm), rows, waves,
+                      self.eps, _lib.stream_ptr())
+            return
         if epi == EPI_ARGMAX and (rope is not None or ring is not None):
             cos, sin, rope_out = rope if rope is not None else (None, None, None)
             host, ctr, err = (tuple(ring) + (None,))[:3] if ring is not None else (None,) * 3
@@ -238,7 +288,7 @@ class Gemv:
                   0 if part is None else part.numel(), M, N, K, epi, int(self.norm), 0, layout,
                   rows, waves, self.eps, _lib.stream_ptr())
 
-    def tune(self, weights, deadline, tiled=None, rounds=3):
+    def tune(self, weights, deadline, tiled=None, rounds=3, given=False):
         """Pick the fastest candidate by GPU time: one call per layer weight (cold),
         captured in a graph and replayed twice (gemv.py:152-195). The candidates'
         graphs are captured first and timed in ``rounds`` interleaved rounds, each
@@ -248,7 +298,9 @@ class Gemv:
         tile_weights copies of ``weights``); without it, tune makes the copies
         itself (before the deadline) and keeps them, so a later call with a
         row-major weight of ``weights`` reads its copy. With the deadline passed
-        nothing is timed and the configuration stays the row-major default."""
+        nothing is timed and the configuration stays the row-major default.
+        ``given``: time layout 5 on an input that the projection before has normalised
+        (``xn``)."""
         dev = weights[0].device
         if any(uses_tiled(c) for c in self.candidates()):
             if tiled is None and time.monotonic() <= deadline:
@@ -262,10 +314,15 @@ class Gemv:
         h = torch.zeros(M, N, device=dev, dtype=BF16)
         ids = torch.zeros(M, device=dev, dtype=torch.int64)
         kw = dict(y=y, nw=nw, h=h, ids=ids)
+        given = given and self.norm and self.epi != EPI_ARGMAX and M <= ROWS_MAX
+
+        def args(cfg):
+            return dict(kw, xn=self.xn_buffer(dev)) if given and cfg[0] == 5 else kw
+
         # the scratch is sized for every candidate before any graph captures it:
         # the graphs are replayed after all captures
         for cfg in self.candidates():
-            if ((self.epi == EPI_ARGMAX or cfg[0] in (3, 4))
+            if ((self.epi == EPI_ARGMAX or cfg[0] in (3, 4, 5))
                     and _lib.lib().ko_gemv_argmax_scratch(self.N, *cfg) > 0):
                 self._scratch(dev, cfg)
         graphs = []
@@ -276,12 +333,12 @@ class Gemv:
             if ws is None:
                 continue
             try:
-                self(x, ws[0], cfg=cfg, **kw)
+                self(x, ws[0], cfg=cfg, **args(cfg))
                 torch.cuda.synchronize()
                 g = torch.cuda.CUDAGraph()
                 with torch.cuda.graph(g):
                     for wt in ws:
-                        self(x, wt, cfg=cfg, **kw)
+                        self(x, wt, cfg=cfg, **args(cfg))
                 g.replay()
                 torch.cuda.synchronize()
             except RuntimeError:

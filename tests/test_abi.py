@@ -155,3 +155,49 @@ def test_prefill_row_kernels_refuse_bad_shapes_without_gpu(libpath):
     assert h.ko_prefill_qkv(*args, 1, 8, 1024, 1024, 1e-6, 32, 8, 64, 8, None) == -95
     assert h.ko_prefill_qkv(*args, 1, 8, 1024, 1022, 1e-6, 32, 8, 128, 8, None) == -22
     assert h.ko_silu_mul2(P, P, P, 12, None) == -22
+
+
+def test_gemv_layout_5_host_rules_without_gpu(libpath):
+    """What layout 5 takes, its scratch, and what ties projections together."""
+    import torch
+    if torch.cuda.device_count() > 0:
+        pytest.skip("fake pointers must not reach a real launch")
+    from kernel_optim_amd import _lib
+    from kernel_optim_amd.kernels import gemv
+    h = _lib.lib()
+    P = 1 << 20
+
+    def call(M, N, K, epi, norm, rows, waves, part_len):
+        return h.ko_gemv(P, P, P, P, None, P, None, P, None, None, None, P, part_len, M, N, K,
+                         epi, norm, 0, 5, rows, waves, 1e-6, None)
+
+    good = [(2560, 4096, 2, 0, 3, 4), (2560, 9728, 2, 0, 3, 4), (2560, 9728, 2, 0, 5, 8),
+            (6144, 2560, 0, 1, 2, 1), (6144, 2560, 1, 1, 2, 1), (9728, 2560, 3, 1, 3, 1),
+            (1000, 2560, 4, 1, 4, 1), (1000, 2560, 4, 1, 6, 1)]
+    for N, K, epi, norm, rows, waves in good:
+        n = h.ko_gemv_argmax_scratch(N, 5, rows, waves)
+        for M in (1, 16, 17, 64, 100):
+            assert call(M, N, K, epi, norm, rows, waves, n) > 0   # a HIP status: no GPU here
+        assert call(4, N, K, epi, norm, rows, waves, n - 1) == -34
+        op = gemv.Gemv(4, N, K, epi, bool(norm))
+        assert (5, rows, waves) in op.rows_cfgs()
+    for N, K, epi, norm, rows, waves in [(2560, 2560, 2, 0, 3, 4), (2558, 4096, 2, 0, 3, 4),
+                                         (8196, 4096, 2, 0, 3, 4), (2560, 4096, 2, 0, 5, 8),
+                                         (2560, 4096, 2, 1, 3, 4), (6144, 2560, 1, 0, 2, 1),
+                                         (6144, 4096, 1, 1, 2, 1), (6144, 2560, 1, 1, 3, 1),
+                                         (9728, 2560, 3, 1, 2, 1), (1000, 2560, 4, 1, 5, 1)]:
+        assert call(4, N, K, epi, norm, rows, waves, 1 << 30) == -95
+        assert (5, rows, waves) not in gemv.Gemv(4, N, K, epi, bool(norm)).rows_cfgs()
+
+    def chained(M, N, K, epi, norm, rows, waves, xn, nw, out):
+        return h.ko_gemv_chained(P, P, P, P, None, P, None, xn, nw, out, P, 1 << 30, M, N, K, epi,
+                                 norm, rows, waves, 1e-6, None)
+
+    assert chained(64, 2560, 4096, 2, 0, 3, 4, None, P, P) > 0
+    assert chained(64, 9728, 2560, 3, 1, 3, 1, P, None, None) > 0
+    assert chained(65, 2560, 4096, 2, 0, 3, 4, None, P, P) == -95    # two weight passes
+    assert chained(4, 2560, 4096, 2, 0, 3, 4, None, None, P) == -22  # no gain
+    assert chained(4, 2560, 4096, 2, 0, 3, 4, P, None, None) == -22  # no norm to replace
+    assert chained(4, 9728, 2560, 3, 1, 3, 1, None, P, P) == -22     # no residual
+    assert chained(4, 196, 4096, 2, 0, 3, 4, None, P, P) == -22      # N % 32
+    assert chained(4, 1000, 2560, 4, 1, 4, 1, P, None, None) == -95  # ARGMAX
