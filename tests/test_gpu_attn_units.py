@@ -1,0 +1,39 @@
+"""One-token attention at the edges of its unit rules."""
+
+import pytest
+import torch
+
+from kernel_optim_amd.kernels.fused import DecodeAttention
+from oracle import attention as A
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def _case(dev, B, cap, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    q = torch.randn(B, 32 * 128, device=dev, generator=g).to(BF)
+    k, v = (torch.randn(B, 8, cap, 128, device=dev, generator=g).to(BF) for _ in range(2))
+    return q, k, v
+
+
+@pytest.mark.parametrize("unit", [64, 32, 16, 1024])
+def test_a_pair_of_one_unit_keeps_the_merged_bits(dev, unit):
+    """Sequences of no key, of one unit (which writes its output itself) and of more in one
+    launch, against the two-launch form (which merges every pair) and the oracle."""
+    cap = 2 * unit + 7
+    lens = [0, 1, 15, 16, unit - 1, unit, unit + 1, cap]
+    q, k, v = _case(dev, len(lens), cap, unit)
+    n = torch.tensor(lens, dtype=torch.int32, device=dev)
+    outs = []
+    for fused in (True, False):
+        op = DecodeAttention(len(lens), 1, cap, 32, 8, 128, dev, unit=unit, fused_combine=fused)
+        out = torch.zeros_like(q)
+        for _ in range(2):   # the counters are left at zero
+            op.with_lengths(q, k, v, n, out)
+        if fused:
+            assert int(op.counters.abs().sum()) == 0
+        outs.append(out)
+    assert torch.equal(outs[0][1:], outs[1][1:])   # nothing is written without a key
+    want = A.decode_attention(q[1:].cpu(), k[1:].cpu(), v[1:].cpu(), lens[1:])
+    torch.testing.assert_close(outs[0][1:].cpu().double(), want, atol=2e-2, rtol=2e-2)
