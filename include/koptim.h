@@ -112,8 +112,8 @@ int ko_decode_attn_token_rows(const void* q, const void* k_cache, const void* v_
  * units_per_seq = 0: units of `unit` keys. units_per_seq = U > 0 (counters
  * given, B <= 64, unit % 64 == 0): each sequence's pos[b] + 1 keys are cut
  * into at most U units of equal size, rounded up to a multiple of 64 and at
- * least `unit` keys, from its length at this step (max_units * unit >= cap
- * still sizes the partials). */
+ * least `unit` keys, from its length at this step, or left whole below 2.5
+ * `unit` keys (max_units * unit >= cap still sizes the partials). */
 int ko_decode_attn_qkv(const void* qkv, const void* q_w, const void* k_w, const void* cos,
                        const void* sin, int max_pos, const int* pos, void* k_cache,
                        void* v_cache, int cap, long long cache_b_stride,

@@ -81,10 +81,14 @@ __device__ __forceinline__ int nunits(int len, int unit) {
   return len > 0 ? (len + unit - 1) / unit : 0;
 }
 // Keys per unit of a sequence of len keys: `unit`, or with usplit > 0 the
-// length cut into usplit parts, rounded up to a multiple of 64, at least `unit`.
+// length cut into usplit parts, rounded up to a multiple of 64, at least `unit`; a
+// sequence of less than 2.5 `unit` is left whole (it then writes its output itself,
+// which is worth more than the second workgroup: 12 sequences of 100 keys 8.6 us in
+// units of 64, 7.3 whole; 40 of 640 keys 32.6 in units of 320, 28.3 whole).
 __device__ __forceinline__ int unit_for(int len, int unit, int usplit) {
   if (usplit <= 0 || len <= 0) return unit;
-  const int u = ((len + usplit - 1) / usplit + 63) & ~63;
+  const int parts = 2 * len < 5 * unit ? 1 : usplit;
+  const int u = ((len + parts - 1) / parts + 63) & ~63;
   return u > unit ? u : unit;
 }
 __device__ __forceinline__ int seq_len(const int* lens, int b, int off, int cap, int rep = 1) {

@@ -169,13 +169,28 @@ def _log(msg):
 
 def attn_units_per_seq(B, nkv):
     """Units per sequence of the one-token decode attention at batch B: at 3..64
-    sequences each sequence's keys are cut at every step into at most
-    256 // (B * nkv) equal units (one round of workgroups over the 256 CUs at
-    equal lengths); at B <= 2 (the attention + o projection launch) fixed units.
-    ENGINE_ATTN_SPLIT >= 0 overrides (0: fixed units)."""
+    sequences each sequence's keys are cut at every step into at most this many equal
+    units; at B <= 2 (the attention + o projection launch) fixed units.
+    One round of workgroups over the 256 CUs at equal lengths, 256 // (B * nkv) units, if
+    that fills them: a lone workgroup takes in about 25 GB/s, whatever the others do (17
+    and 32 sequences of 1024 keys: 25.7 and 28.8 us on 136 and 256 workgroups). Where it
+    leaves 15 % or more of the CUs idle, the cut into at most 3 units (up to 16 sequences:
+    512 units in all) that fills its rounds best: 12 sequences of 2048 keys 29.5 -> 26.8
+    us (2 -> 5 units), 18 45.1 -> 37.0 (1 -> 3), 40 79.5 -> 71.4 (1 -> 3), 48 87.1 -> 78.7
+    (1 -> 2). ENGINE_ATTN_SPLIT >= 0 overrides (0: fixed units)."""
     if ATTN_SPLIT >= 0:
         return ATTN_SPLIT
-    return max(1, 256 // (B * nkv)) if 3 <= B <= 64 else 0
+    if not 3 <= B <= 64:
+        return 0
+
+    def fill(u):   # the share of its rounds' CUs that have a workgroup
+        n = B * nkv * u
+        return n / (-(-n // 256) * 256)
+
+    base = max(1, 256 // (B * nkv))
+    more = range(base + 1, (512 // (B * nkv) if B <= 16 else min(3, 1024 // (B * nkv))) + 1)
+    best = max(more, key=fill, default=base)
+    return best if fill(best) >= fill(base) + 0.15 else base
 
 
 def rows_served(cfg):

@@ -113,14 +113,18 @@ class DecodeAttention:
         self.token_rows = bool(token_rows)
         # units_per_seq = U > 0: decode_qkv cuts each sequence's keys into at most U
         # equal units (multiples of 64 keys, at least `unit`) from its length at
-        # each step, so a batch of equal lengths fills one round of the grid
-        # whatever the position (ko_decode_attn_qkv)
+        # each step, so a batch of equal lengths fills whole rounds of the grid
+        # whatever the position; less than 2.5 `unit` keys stay whole
+        # (ko_decode_attn_qkv)
         self.units_per_seq = int(units_per_seq)
         if self.units_per_seq:
             _need(self.units_per_seq > 0 and T == 1 and not self.token_rows and fused_combine
                   and B <= 64, "units_per_seq serves one token per sequence, B <= 64, with "
                   "the fused combine")
-            unit = 64 if unit is None else unit
+            if unit is None:
+                # the smallest unit: two workgroups on a CU gain less from short ones
+                one_round = B * nkv * self.units_per_seq <= 256
+                unit = 64 if one_round else 128 if B <= 16 else 320
             _need(unit % 64 == 0, "units_per_seq needs a unit (the smallest unit) % 64 == 0")
         _need(unit is None or (unit % 16 == 0 and unit >= 16),
               "unit must be a positive multiple of 16")

@@ -52,3 +52,17 @@ def test_accept_prefix_and_next_token():
 
 def test_draft_len_by_batch():
     assert [draft_len(b) for b in (1, 4, 5, 16, 17, 32, 33)] == [6, 6, 4, 4, 2, 2, 0]
+
+
+def test_attention_units_per_sequence_fill_the_cus():
+    """One round of the 256 CUs where that fills them, else the cut that fills its rounds
+    best; fixed units for one or two sequences and above 64."""
+    from kernel_optim_amd.engine import attn_units_per_seq
+    assert [attn_units_per_seq(B, 8) for B in (1, 2, 3, 4, 8, 10, 16, 32, 64, 65)] == \
+        [0, 0, 10, 8, 4, 3, 2, 1, 1, 0]
+    assert [attn_units_per_seq(B, 8) for B in (11, 12, 13, 17, 21, 22, 24, 33, 42, 43, 48, 49)] == \
+        [5, 5, 2, 3, 3, 1, 1, 3, 3, 2, 2, 1]
+    for nkv in (1, 2, 8):
+        for B in range(3, 65):
+            u = attn_units_per_seq(B, nkv)
+            assert u >= 1 and B * nkv * u <= 1024

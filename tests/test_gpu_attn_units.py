@@ -37,3 +37,29 @@ def test_a_pair_of_one_unit_keeps_the_merged_bits(dev, unit):
     assert torch.equal(outs[0][1:], outs[1][1:])   # nothing is written without a key
     want = A.decode_attention(q[1:].cpu(), k[1:].cpu(), v[1:].cpu(), lens[1:])
     torch.testing.assert_close(outs[0][1:].cpu().double(), want, atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("split,unit", [(1, 64), (2, None), (3, 320), (5, 128), (10, None)])
+def test_per_sequence_units(dev, split, unit):
+    """decode_qkv cutting each sequence by its own length: lengths on both sides of the
+    one that is left whole (2.5 units), of the smallest unit and of whole units."""
+    u = unit or 64
+    lens = [1, 63, 64, 65, (5 * u - 1) // 2, 5 * u // 2, 5 * u // 2 + 1, u * split, u * split + 1,
+            2 * u * split + 3]
+    B, cap = len(lens), -(-max(lens) // 16) * 16
+    q, k, v = _case(dev, B, cap, split)
+    g = torch.Generator(device=dev).manual_seed(7)
+    qkv = torch.randn(B, 48 * 128, device=dev, generator=g).to(BF)
+    ones = torch.ones(128, dtype=BF, device=dev)
+    cos, sin = torch.ones(cap, 128, dtype=BF, device=dev), torch.zeros(cap, 128, dtype=BF, device=dev)
+    pos = torch.tensor(lens, dtype=torch.int32, device=dev) - 1
+    op = DecodeAttention(B, 1, cap, 32, 8, 128, dev, unit=unit, fused_combine=True,
+                         units_per_seq=split)
+    out = torch.zeros_like(q)
+    for _ in range(2):
+        op.decode_qkv(qkv, ones, ones, cos, sin, pos, k, v, out, 1e-6)
+    assert int(op.counters.abs().sum()) == 0
+    from kernel_optim_amd.prefill import rmsnorm   # cos = 1, sin = 0: the norm alone
+    qn = rmsnorm(qkv[:, :32 * 128].view(B, 32, 128), ones, 1e-6).view(B, -1)
+    want = A.decode_attention(qn.cpu(), k.cpu(), v.cpu(), lens)
+    torch.testing.assert_close(out.cpu().double(), want, atol=2e-2, rtol=2e-2)
