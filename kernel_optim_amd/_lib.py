@@ -9,6 +9,8 @@ status. There is no fallback: if the library is missing, using an op raises.
 import ctypes
 import os
 
+import torch
+
 from .build import LIB_PATH
 
 _c_void_p = ctypes.c_void_p
@@ -104,7 +106,7 @@ def status_message(code):
 
 
 def call(name, *args):
-    st = getattr(lib(), name)(*args)
+    st = getattr(_lib or lib(), name)(*args)
     if st != 0:
         raise RuntimeError(f"{name} failed: {status_message(st)} (status {st})")
 
@@ -137,5 +139,9 @@ def host_device_ptr(t):
 
 
 def stream_ptr(device=None):
-    import torch
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle (through torch's raw accessor where it has one:
+    0.2 us, against 0.9 us with a Stream object built per call)."""
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None or device is not None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return raw(torch.cuda.current_device())

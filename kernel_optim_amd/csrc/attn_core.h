@@ -727,6 +727,25 @@ __device__ __forceinline__ void attn1_body(const AttnArgs& a, int wg, int nwg,
     }
     __syncthreads();  // the next unit reuses the LDS
   }
+  // A sequence without keys has no unit: its output rows are zeros, as the second
+  // launch's merge of no slots writes them (the QKV prologue always appends a key).
+  if constexpr (FUSED && !QKV) {
+    auto zero = [&](int b) {
+      uint32_t* ob = reinterpret_cast<uint32_t*>(a.out + (long long)b * nq * D);
+      for (int i = threadIdx.x; i < nq * D / 2; i += 64 * WM) ob[i] = 0u;
+    };
+    if (a.B == 1) {
+      if (total == 0 && wg == 0) zero(0);
+    } else if (small_b) {
+      for (unsigned long long m = __ballot(lane < a.B && my_len <= 0); m; m &= m - 1) {
+        const int b = __builtin_ctzll(m);
+        if (b % nwg == wg) zero(b);
+      }
+    } else {
+      for (int b = wg; b < a.B; b += nwg)
+        if (seq_len(a.lens, b, a.len_off, a.cap, a.rep) <= 0) zero(b);
+    }
+  }
   hooks.end();
 }
 

@@ -650,16 +650,23 @@ class Engine:
     def verify_step(self, rows, pos):
         """Replay the verify graph for rows [B, K+1] (int64: the last accepted token
         and K drafts) at positions pos [B] (of rows[:, 0]); returns the greedy ids
-        [B, K+1] and, with keep_logits, the bf16 logits [B*(K+1), V], on the CPU.
-        Writes K/V cache slots pos .. pos+K. Needs a setup with speculation."""
+        [B, K+1] and, with keep_logits, the bf16 logits [B*(K+1), V], on the CPU
+        (in pinned memory: 2 MB of logits arrive in 50 us, against 190-480 us through
+        a pageable tensor). Writes K/V cache slots pos .. pos+K. Needs a setup with
+        speculation."""
         if self.gk is None:
             raise ValueError("verify_step needs an engine set up with speculation (spec=True, "
                              "max_new_tokens > 2, a batch of at most 32)")
-        self.vin.copy_(torch.as_tensor(rows, dtype=torch.int64))
-        self._set_pos(torch.as_tensor(pos, dtype=torch.int32).to(DEVICE))
+        # nothing in flight reads the pinned inputs: every user of them waits for its step
+        self.pin_vin.copy_(torch.as_tensor(rows, dtype=torch.int64))
+        self.pin_pos.copy_(torch.as_tensor(pos, dtype=torch.int32))
+        self.vin.copy_(self.pin_vin, non_blocking=True)
+        self._set_pos(self.pin_pos)
         self.gk.replay()
+        out = [torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t, non_blocking=True)
+               for t in ((self.vout, self.logitsT) if self.keep_logits else (self.vout,))]
         torch.cuda.synchronize()
-        return self.vout.cpu(), (self.logitsT.cpu() if self.keep_logits else None)
+        return out[0], (out[1] if self.keep_logits else None)
 
     @torch.inference_mode()
     def time_step(self, reps=20):

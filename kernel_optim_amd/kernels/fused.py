@@ -42,6 +42,13 @@ def _check(t, name, dtype, shape=None, contiguous=True):
         _need(t.is_contiguous(), f"{name} must be contiguous")
 
 
+def _is(t, dtype, shape):
+    """_check's conditions as one test, for calls that are made per token and layer: the
+    caller falls back on _check, which names what is wrong."""
+    return (isinstance(t, torch.Tensor) and t.dtype is dtype and t.is_cuda and t.shape == shape
+            and t.is_contiguous())
+
+
 def _check_cache(t, name, B, nkv, cap, d):
     _need(t.dim() == 4, f"{name} must be [B, nkv, cap, d]")
     _need(tuple(t.shape) == (B, nkv, cap, d), f"{name} must have shape {(B, nkv, cap, d)}, got {tuple(t.shape)}")
@@ -91,8 +98,8 @@ class DecodeAttention:
     shared by the 4 wavefronts of a workgroup (merged in LDS), so the unit is
     4x the per-wavefront share.
 
-    A second launch merges the partials, as the reference does; with
-    ``fused_combine`` the last unit of each (sequence, KV head) merges them in
+    A second launch merges the partials, as the reference does, where the units take
+    several rounds of the grid; with one round, or ``fused_combine``, the last unit of each (sequence, KV head) merges them in
     the same launch instead, through an arrival counter. The partials and the
     counter travel through device-coherent stores, loads and atomics (no fence,
     no L2 write-back).
@@ -133,20 +140,29 @@ class DecodeAttention:
         rows = B * T * nq
         self.o_part = torch.empty(rows * self.max_units * d, dtype=torch.float32, device=device)
         self.ml = torch.empty(rows * self.max_units * 2, dtype=torch.float32, device=device)
-        # per-(sequence or token row, KV head) arrival counters; every launch leaves
-        # them at zero
+        # Words that start at zero, from one allocation: per-(sequence or token row, KV
+        # head) arrival counters, which every launch leaves at zero; decode_qkv_oproj's
+        # counters and done flags, and its wait-failure flag.
         rows_k = B * T if self.token_rows else B  # rows of the one-token kernel
-        self.counters = (torch.zeros(rows_k * nkv, dtype=torch.int32, device=device)
-                         if fused_combine else None)
-        # decode_qkv_oproj: its counters and done flags, and its wait-failure flag
-        self.sync = torch.zeros(_lib.lib().ko_decode_attn_qkv_oproj_sync_ints(), dtype=torch.int32,
-                                device=device)
-        self.err = torch.zeros(1, dtype=torch.int32, device=device)
+        n_sync = _lib.lib().ko_decode_attn_qkv_oproj_sync_ints()
+        words = torch.zeros(n_sync + 4 + rows_k * nkv, dtype=torch.int32, device=device)
+        self.sync, self.err = words[:n_sync], words[n_sync:n_sync + 1]
+        self.counters = words[n_sync + 4:] if fused_combine else None
+        # The two-launch form of one query token whose units are one round of the grid
+        # merges in its one launch too, on these counters: the bits of two launches (B = 1,
+        # 512 keys: 8.9 -> 7.2 us; 4 x 2048 15.1 -> 13.1; 16 x 8192 83.6 -> 81.4).
+        # Several rounds stay with two launches (ragged B = 64 5,887 against 5,771 GB/s).
+        one_round = B * nkv * self.max_units * self.waves_per_unit <= self.grid_waves
+        self._own_counters = (words[n_sync + 4:] if T == 1 and not fused_combine and one_round
+                              else None)
         self.oproj_delay_ns = 1000
         # polls of a pair's done flag before a decode_qkv_oproj wait gives up and
         # sets err (-1: the library's bound; 0: give up at once, for tests)
         self.oproj_spin = -1
         self.scale = d ** -0.5
+        self._q_shape = torch.Size((B * T, nq * d))
+        self._kv_shape = torch.Size((B, nkv, cap, d))
+        self._len_shape = torch.Size((B,))
 
     def _check_kv(self, k_cache, v_cache, lens):
         B, nkv, d, cap = self.B, self.nkv, self.d, self.cap
@@ -156,15 +172,23 @@ class DecodeAttention:
         _check(lens, "pos/lengths", torch.int32, (B,))
 
     def _run(self, q, k_cache, v_cache, lens, len_offset, out):
-        B, T, nq, nkv, d, cap = self.B, self.T, self.nq, self.nkv, self.d, self.cap
-        _check(q, "q", BF16, (B * T, nq * d))
-        _check(out, "out", BF16, (B * T, nq * d))
-        self._check_kv(k_cache, v_cache, lens)
-        _lib.call("ko_decode_attn", _lib.ptr(q), _lib.ptr(k_cache), _lib.ptr(v_cache),
-                  _lib.ptr(lens), len_offset, cap, k_cache.stride(0), k_cache.stride(1),
-                  B, T, nkv, d, self.unit, self.max_units, self.grid_waves, self.scale,
-                  _lib.ptr(self.o_part), _lib.ptr(self.ml), _lib.ptr(self.counters),
-                  _lib.ptr(out), _lib.stream_ptr())
+        strides = k_cache.stride() if isinstance(k_cache, torch.Tensor) else None
+        if not (_is(q, BF16, self._q_shape) and _is(out, BF16, self._q_shape)
+                and _is(lens, torch.int32, self._len_shape)
+                and isinstance(v_cache, torch.Tensor) and strides == v_cache.stride()
+                and k_cache.shape == self._kv_shape == v_cache.shape
+                and strides[2:] == (self.d, 1)
+                and k_cache.dtype is BF16 and v_cache.dtype is BF16
+                and k_cache.is_cuda and v_cache.is_cuda):
+            _check(q, "q", BF16, self._q_shape)
+            _check(out, "out", BF16, self._q_shape)
+            self._check_kv(k_cache, v_cache, lens)
+        counters = self.counters if self.counters is not None else self._own_counters
+        _lib.call("ko_decode_attn", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                  lens.data_ptr(), len_offset, self.cap, strides[0], strides[1], self.B, self.T,
+                  self.nkv, self.d, self.unit, self.max_units, self.grid_waves, self.scale,
+                  self.o_part.data_ptr(), self.ml.data_ptr(), _lib.ptr(counters), out.data_ptr(),
+                  _lib.stream_ptr())
 
     def __call__(self, q, k_cache, v_cache, pos, out):
         """q: [B*T, NQ*D]; k/v_cache: [B, NKV, cap, D]; pos: [B] int32 (first query

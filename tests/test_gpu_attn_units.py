@@ -26,15 +26,19 @@ def test_a_pair_of_one_unit_keeps_the_merged_bits(dev, unit):
     q, k, v = _case(dev, len(lens), cap, unit)
     n = torch.tensor(lens, dtype=torch.int32, device=dev)
     outs = []
-    for fused in (True, False):
-        op = DecodeAttention(len(lens), 1, cap, 32, 8, 128, dev, unit=unit, fused_combine=fused)
-        out = torch.zeros_like(q)
+    for fused in (True, False, None):   # one launch asked for, two launches, one by the op's rule
+        op = DecodeAttention(len(lens), 1, cap, 32, 8, 128, dev, unit=unit,
+                             fused_combine=bool(fused))
+        if fused is False:
+            op._own_counters = None
+        out = torch.full_like(q, float("nan"))
         for _ in range(2):   # the counters are left at zero
             op.with_lengths(q, k, v, n, out)
-        if fused:
-            assert int(op.counters.abs().sum()) == 0
+        for c in (op.counters, op._own_counters):
+            assert c is None or int(c.abs().sum()) == 0
         outs.append(out)
-    assert torch.equal(outs[0][1:], outs[1][1:])   # nothing is written without a key
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[2], outs[1])
+    assert int(outs[0][0].float().abs().sum()) == 0   # no key: zeros
     want = A.decode_attention(q[1:].cpu(), k[1:].cpu(), v[1:].cpu(), lens[1:])
     torch.testing.assert_close(outs[0][1:].cpu().double(), want, atol=2e-2, rtol=2e-2)
 
@@ -63,3 +67,36 @@ def test_per_sequence_units(dev, split, unit):
     qn = rmsnorm(qkv[:, :32 * 128].view(B, 32, 128), ones, 1e-6).view(B, -1)
     want = A.decode_attention(qn.cpu(), k.cpu(), v.cpu(), lens)
     torch.testing.assert_close(out.cpu().double(), want, atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("B,lens", [(1, [0]), (70, [0, 5] * 35)])
+def test_sequences_without_keys_give_zeros(dev, B, lens):
+    """One sequence, and more than 64 (whose lengths are read in chunks)."""
+    q, k, v = _case(dev, B, 16, B)
+    n = torch.tensor(lens, dtype=torch.int32, device=dev)
+    outs = []
+    for own in (True, False):
+        op = DecodeAttention(B, 1, 16, 32, 8, 128, dev, unit=16)
+        assert op._own_counters is not None
+        op._own_counters = op._own_counters if own else None
+        out = torch.full_like(q, float("nan"))
+        op.with_lengths(q, k, v, n, out)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
+    assert int(outs[0][0].float().abs().sum()) == 0
+
+
+def test_bad_arguments_are_named(dev):
+    q, k, v = _case(dev, 2, 32, 1)
+    n = torch.tensor([3, 4], dtype=torch.int32, device=dev)
+    op = DecodeAttention(2, 1, 32, 32, 8, 128, dev)
+    out = torch.zeros_like(q)
+    bad = [("q must have shape", (q[:1], k, v, n, out)), ("out must be torch.bf", (q, k, v, n, out.float())),
+           ("must share strides", (q, k, v.transpose(0, 1).contiguous().transpose(0, 1), n, out)),
+           ("must have shape", (q, k[:, :, :16], v, n, out)), ("int32", (q, k, v, n.long(), out)),
+           ("must be contiguous", (q, k, v, n, torch.zeros(4096, 2, dtype=BF, device=dev).t())),
+           ("on the GPU", (q.cpu(), k, v, n, out)), ("must be a tensor", (None, k, v, n, out)),
+           ("bf16 GPU", (q, k.float(), v.float(), n, out))]
+    for text, args in bad:
+        with pytest.raises(ValueError, match=text):
+            op.with_lengths(*args)
