@@ -40,6 +40,14 @@ __global__ __launch_bounds__(64 * WPG) void gemv_mfma_kernel(GemvArgs a, int nti
   static_assert(MT == 1 || (MT == 2 && WPG * 64 >= 512), "16 or 32 rows of x");
   constexpr int NW = EPI == EPI_SWIGLU ? 2 : 1;
   constexpr bool HPRE = EPI == EPI_RESID && S <= 16;  // residual loaded ahead (registers)
+  // One row tile: x goes to the operand order through LDS (XL), loaded in runs of a row's
+  // 4 S 16-byte chunks, as many loads as the rows hold; read straight into that order
+  // every load touches 16 rows, half a line each (and one memory channel of 16, at the o
+  // projection's row length): 16 / 4 rows, o 8.46 -> 6.66 / 6.67 -> 5.87 us, qkv 9.77 ->
+  // 9.10 / 8.69 -> 8.47.
+  constexpr bool XL = MT == 1 && S <= 16;
+  constexpr int CPR = 4 * S;  // chunks of a row in a wavefront's K slice
+  __shared__ uint4 s_x[XL ? WPG : 1][XL ? S * 68 : 1];
   __shared__ float s_c[WPG][NW][16 * MT][17];
   __shared__ float s_sq[WPG][16 * MT];
 
@@ -66,20 +74,24 @@ __global__ __launch_bounds__(64 * WPG) void gemv_mfma_kernel(GemvArgs a, int nti
   // NORM gain) is loaded first, then the first tile's weights: loads return in
   // issue order, so the prologue runs while the weights stream. The weights
   // stay issued there (the scheduler would otherwise sink the loads next to
-  // their MFMAs to save registers). With NORM the compiler turns the masked x
-  // loads into branches and waits for the second one before issuing the rest,
-  // so the weights go out one memory round trip after x. Measured at 16 rows,
-  // that order beats issuing everything at once (unmasked loads: qkv 10.5
-  // against 10.3 us, gate/up 20.7 against 20.1) and an explicit wait for all
-  // of x and the gain before the weights (10.4 / 20.7).
+  // their MFMAs to save registers).
   constexpr bool NW_EARLY = NORM && S <= 10;
   bf16x8 xa[S];
   bf16x8 xa2[MT > 1 ? S : 1];  // MT = 2: rows 16..31 of x, the A operand of a second MFMA
   {
     const uint16_t* xrow = a.x + (long long)(mok ? col : 0) * K + kw0;
     uint4 xr[S], nwv[NW_EARLY ? S : 1], xr2[MT > 1 ? S : 1];
+    if constexpr (XL) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) xr[s] = mok ? ldg16(xrow + 32 * s) : make_uint4(0, 0, 0, 0);
+      for (int i = 0; i < S; ++i) {
+        const int c = 64 * i + lane, row = c / CPR;
+        if (64 * i < mr * CPR)  // uniform; rows past mrows stay undefined, and so unused
+          xr[i] = ldg16(a.x + (long long)min(row, mr - 1) * K + wv * (32 * S) + 8 * (c - row * CPR));
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < S; ++s) xr[s] = mok ? ldg16(xrow + 32 * s) : make_uint4(0, 0, 0, 0);
+    }
     if constexpr (MT > 1) {
       const uint16_t* xrow2 = a.x + (long long)(mok2 ? col + 16 : 0) * K + kw0;
 #pragma unroll
@@ -102,6 +114,20 @@ __global__ __launch_bounds__(64 * WPG) void gemv_mfma_kernel(GemvArgs a, int nti
 #pragma unroll
     for (int s = 0; s < PD; ++s) issue(blockIdx.x, s, s);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (XL) {
+      // chunk kc of row m at 68 (kc / 4) + 17 (kc % 4) + m: stores of consecutive chunks
+      // and loads of consecutive rows both step through the banks
+#pragma unroll
+      for (int i = 0; i < S; ++i) {
+        const int c = 64 * i + lane, row = c / CPR, kc = c - row * CPR;
+        if (64 * i < mr * CPR) s_x[wv][68 * (kc >> 2) + 17 * (kc & 3) + row] = xr[i];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int s = 0; s < S; ++s) xr[s] = s_x[wv][68 * s + 17 * g + col];
+    }
     if constexpr (NORM) {
       float rstd, rstd2 = 0.f;
       if (a.ss) {

@@ -166,3 +166,25 @@ def test_layouts_of_one_projection_may_alternate(dev):
         h = h0.clone()
         op(x, Wt, h=h, cfg=cfg)
         assert_resid_close(h.cpu(), want, y)
+
+
+@pytest.mark.parametrize("K", [2560, 4096])
+@pytest.mark.parametrize("M", [1, 2, 3, 5, 8, 13, 15, 16])
+def test_layout_2_takes_x_in_row_runs(dev, M, K):
+    """Layout 2 loads a wavefront's slice of x as runs of its rows and only as many loads as
+    the rows hold; rows past M (poisoned here) reach no output."""
+    N = 1000
+    g = _g(dev, M)
+    buf = torch.full((M + 1, K), float("nan"), device=dev, dtype=BF)
+    x = buf[:M]
+    x.copy_(torch.randn(M, K, device=dev, generator=g))
+    nw = (1 + 0.1 * torch.randn(K, device=dev, generator=g)).to(BF)
+    W = _w(dev, N, K, 3)
+    Wt = gemv.tile_weights(W)
+    for norm in (False, True):
+        kw = dict(nw=nw, ss=None) if norm else {}
+        y = torch.empty(M, N, device=dev)
+        gemv.Gemv(M, N, K, gemv.EPI_F32, norm=norm)(x, Wt, y=y, cfg=(2, 1, 0), **kw)
+        ref = dict(nw=nw.cpu(), ss=x.cpu().float().pow(2).sum(-1)) if norm else {}
+        want = O.gemv(x.cpu(), W.cpu(), O.EPI_F32, **ref)
+        torch.testing.assert_close(y.cpu(), want, rtol=2e-3, atol=2e-3)
