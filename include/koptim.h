@@ -282,9 +282,9 @@ int ko_embed_ss(const long long* ids, const void* emb, void* h, float* ss, int M
  *           column tiles per workgroup, K in `waves` slices. Behind a norm (norm
  *           != 0, K = 2560, `waves` 1): F32 or BF16 with `rows` 2, SWIGLU 3,
  *           ARGMAX 4 or 6; x is normalised by a launch of its own. RESID without
- *           a norm (N % 4 == 0, N <= 8192): `rows` 3 in 4 slices (K = 4096,
- *           9728) or 5 in 8 (K = 9728); a second launch adds the slices' fp32
- *           sums in slice order (deterministic) and the residual. part is its
+ *           a norm (N % 4 == 0, N <= 8192, K = 4096 or 9728): `rows` 3, `waves`
+ *           4; a second launch adds the slices' fp32 sums in slice order
+ *           (deterministic) and the residual. part is its
  *           scratch (part_len >= ko_gemv_argmax_scratch(N, 5, rows, waves));
  *           calls that share it must not overlap.
  * K % 8 == 0. M larger than a slice is processed in several launches. */

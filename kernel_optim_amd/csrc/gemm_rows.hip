@@ -13,9 +13,9 @@
 //     into slices with plain stores of the fp32 sums; row_finish_kernel adds them,
 //     the residual, and leaves the next projection's normalised x.
 // Measured against layouts 2 and 4 with their norms (us, cold weights; the residual
-// projections with their row_finish): 32 rows qkv 14.3 -> 9.2, o 10.5 -> 9.7, gate/up 24.3
-// -> 20.5, down 19.5 -> 15.1; 64 rows 27.7 -> 12.0, 15.5 -> 12.1, 47.5 -> 24.7, 31.9 ->
-// 19.2; a norm of its own costs 2.8-3.6.
+// projections with their row_finish): 32 rows qkv 14.3 -> 9.2, o 10.5 -> 8.9, gate/up 24.3
+// -> 20.5, down 19.5 -> 14.0; 64 rows 27.7 -> 12.0, 15.5 -> 10.5, 47.5 -> 24.7, 31.9 ->
+// 17.2; a norm of its own costs 2.8-3.6.
 #include "gemv_launch.h"
 
 using namespace ko;
@@ -39,44 +39,82 @@ __device__ __forceinline__ long long xt_index(int m, int k, int mt) {
 }
 
 // Workgroup (group, slice): TN column tiles (with their up tiles for SWIGLU) over the
-// slice's `steps` K steps of 32, dealt out to the wavefronts one step at a time (NS =
-// steps / 8, rounded up). A wavefront multiplies every weight block of a step with all MT
-// row tiles of x; x and weights run through one ring of PD steps in registers (as many
-// as they hold beside MT * NB accumulators). XT: x in the operand order, padded to 16 MT
-// rows. SUMS: the slice's fp32 sums to part[slice][row][column], else the epilogue.
+// slice's `steps` K steps of 32, at most NS a wavefront. A wavefront multiplies every
+// weight block of a step with all MT row tiles of x. SUMS: the slice's fp32 sums to
+// part[slice][row][column], else the epilogue.
+// XT: x in the operand order, padded to 16 MT rows; the steps are dealt out one at a time,
+// and x and weights run through one ring of PD steps in registers (as many as they hold
+// beside MT * NB accumulators). Else x in rows: a wavefront has consecutive steps, loads
+// their x as runs of each row, turns it through its own LDS (as layout 2) and keeps it;
+// only the weights run through the ring (64 / 32 rows, against x read from rows in operand
+// order in the ring: o 13.1 -> 10.5 / 10.1 -> 8.9 us, down 20.2 -> 17.2 / 15.1 -> 14.0).
 template <int EPI, bool XT, bool SUMS, int MT, int TN, int NS, int PD>
 __global__ __launch_bounds__(64 * RW, 1) void gemm_rows_kernel(GemvArgs a, int nslices, int steps,
                                                                float* __restrict__ part) {
   constexpr int NW = EPI == EPI_SWIGLU ? 2 : 1, NB = TN * NW;
   constexpr int MR = NB * MT <= 12 ? MT : 12 / NB;  // row tiles summed per round (96 KiB)
   static_assert(MR >= 1 && PD <= NS, "one row tile of sums fits the LDS");
-  __shared__ float4 s_c[RW][MR * NB][64];
+  // a wavefront's own region: its x on the way to the operand order, later its sums
+  constexpr int XR = XT ? 0 : 68 * NS, CR = MR * NB * 64, CPR = 4 * NS;
+  __shared__ uint4 s_w[RW][XR > CR ? XR : CR];
   __shared__ float2 s_best[EPI == EPI_ARGMAX ? MT * 16 : 1][TN];
   const int t = threadIdx.x, wv = t >> 6, lane = t & 63, col = lane & 15, g = lane >> 4;
   const int N = a.N, K = a.K, mr = a.mrows, T = (N + 15) / 16, KS = K / 32;
   const int group = blockIdx.x / nslices, slice = blockIdx.x - group * nslices;
   const int s0 = slice * steps, tile0 = group * TN;
+  // step j of this wavefront: first + stride * j, while below `steps`
+  const int first = XT ? wv : wv * NS;
+  constexpr int STRIDE = XT ? RW : 1;
 
-  const uint16_t* xp[MT];
-#pragma unroll
-  for (int u = 0; u < MT; ++u)  // rows past mrows: a valid row, whose result is not used
-    xp[u] = XT ? a.x + (u * 64 + lane) * 8
-               : a.x + (long long)min(16 * u + col, mr - 1) * K + 8 * g;
   const uint16_t* wp[NB];
 #pragma unroll
   for (int n = 0; n < NB; ++n)
     wp[n] = a.w + ((long long)min(tile0 + n / NW, T - 1) + (n % NW) * T) * KS * 512 + 8 * lane;
-  uint4 xb[PD][MT], wb[PD][NB];
+  uint4 xb[XT ? PD : NS][MT], wb[PD][NB];
   auto issue = [&](int j, int slot) {
-    const int st = s0 + min(wv + RW * j, steps - 1);  // past the end: loaded, not used
+    const int st = s0 + min(first + STRIDE * j, steps - 1);  // past the end: loaded, not used
+    if constexpr (XT) {
 #pragma unroll
-    for (int u = 0; u < MT; ++u) xb[slot][u] = ldg16(xp[u] + (long long)st * (XT ? MT * 512 : 32));
+      for (int u = 0; u < MT; ++u)
+        xb[slot][u] = ldg16(a.x + ((long long)st * MT + u) * 512 + 8 * lane);
+    }
 #pragma unroll
     for (int n = 0; n < NB; ++n) wb[slot][n] = ldg16_stream(wp[n] + (long long)st * 512);
   };
+  if constexpr (!XT) {
+    // rows past mrows and steps past the slice: a valid chunk, whose result is not used
+    const int kmax = 4 * max(min(steps - first, NS), 1) - 1;
+    const uint16_t* xs = a.x + (s0 + min(first, steps - 1)) * 32;
+#pragma unroll
+    for (int u = 0; u < MT; ++u)
+#pragma unroll
+      for (int i = 0; i < NS; ++i) {
+        const int ch = 64 * i + lane, row = ch / CPR, kc = min(ch - row * CPR, kmax);
+        if (64 * i < (mr - 16 * u) * CPR)  // uniform
+          xb[i][u] = ldg16(xs + (long long)min(16 * u + row, mr - 1) * K + 8 * kc);
+      }
+    __builtin_amdgcn_sched_barrier(0);  // x ahead of the weights: loads return in order
+  }
 #pragma unroll
   for (int j = 0; j < PD; ++j) issue(j, j);
   __builtin_amdgcn_sched_barrier(0);  // the whole ring is in flight before the first product
+  if constexpr (!XT) {
+#pragma unroll
+    for (int u = 0; u < MT; ++u) {
+#pragma unroll
+      for (int i = 0; i < NS; ++i) {
+        const int ch = 64 * i + lane, row = ch / CPR, kc = ch - row * CPR;
+        if (64 * i < (mr - 16 * u) * CPR) s_w[wv][68 * (kc >> 2) + 17 * (kc & 3) + row] = xb[i][u];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int j = 0; j < NS; ++j) xb[j][u] = s_w[wv][68 * j + 17 * g + col];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
 
   f32x4 c[MT][NB];
 #pragma unroll
@@ -86,13 +124,14 @@ __global__ __launch_bounds__(64 * RW, 1) void gemm_rows_kernel(GemvArgs a, int n
 #pragma unroll
   for (int j = 0; j < NS; ++j) {
     const int slot = j % PD;
-    if (wv + RW * j < steps) {  // uniform per wavefront
+    if (first + STRIDE * j < steps) {  // uniform per wavefront
 #pragma unroll
       for (int n = 0; n < NB; ++n)
 #pragma unroll
         for (int u = 0; u < MT; ++u)
           c[u][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8, xb[slot][u]), __builtin_bit_cast(bf16x8, wb[slot][n]),
+              __builtin_bit_cast(bf16x8, xb[XT ? slot : j][u]),
+              __builtin_bit_cast(bf16x8, wb[slot][n]),
               c[u][n], 0, 0, 0);
     }
     if (j + PD < NS) issue(j + PD, slot);
@@ -108,7 +147,7 @@ __global__ __launch_bounds__(64 * RW, 1) void gemm_rows_kernel(GemvArgs a, int n
     for (int u = u0; u < u0 + MR && u < MT; ++u)
 #pragma unroll
       for (int n = 0; n < NB; ++n)
-        s_c[wv][(u - u0) * NB + n][lane] = make_float4(c[u][n][0], c[u][n][1], c[u][n][2], c[u][n][3]);
+        s_w[wv][((u - u0) * NB + n) * 64 + lane] = __builtin_bit_cast(uint4, c[u][n]);
     __syncthreads();
     const int ru = min(MR, MT - u0);
     for (int task = wv; task < ru * TN; task += RW) {
@@ -116,11 +155,11 @@ __global__ __launch_bounds__(64 * RW, 1) void gemm_rows_kernel(GemvArgs a, int n
       float tot[4] = {0.f, 0.f, 0.f, 0.f}, tot2[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int w = 0; w < RW; ++w) {
-        const float4 v = s_c[w][u * NB + q * NW][lane];
-        tot[0] += v.x, tot[1] += v.y, tot[2] += v.z, tot[3] += v.w;
+        const f32x4 v = __builtin_bit_cast(f32x4, s_w[w][(u * NB + q * NW) * 64 + lane]);
+        tot[0] += v[0], tot[1] += v[1], tot[2] += v[2], tot[3] += v[3];
         if constexpr (NW == 2) {
-          const float4 v2 = s_c[w][u * NB + q * NW + 1][lane];
-          tot2[0] += v2.x, tot2[1] += v2.y, tot2[2] += v2.z, tot2[3] += v2.w;
+          const f32x4 v2 = __builtin_bit_cast(f32x4, s_w[w][(u * NB + q * NW + 1) * 64 + lane]);
+          tot2[0] += v2[0], tot2[1] += v2[1], tot2[2] += v2[2], tot2[3] += v2[3];
         }
       }
       const int n = (tile0 + q) * 16 + col;
@@ -275,18 +314,11 @@ namespace ko {
 int launch_layout5(GemvArgs a, int epi, bool norm, int tn, int slices, const RowsChain& chain,
                    float* part, hipStream_t s) {
   if (epi == EPI_RESID) {
-    int st;
-    if (a.K == 4096 && slices == 4)
-      st = go_mt<EPI_RESID, false, true, 3, 4, 4, 4, 4, 4>(a, slices, part, s);
-    else if (a.K == 9728 && slices == 4)
-      st = go_mt<EPI_RESID, false, true, 3, 10, 8, 8, 6, 5>(a, slices, part, s);
-    else
-      st = go_mt<EPI_RESID, false, true, 5, 5, 5, 5, 4, 4>(a, slices, part, s);
+    int st = a.K == 4096 ? go_mt<EPI_RESID, false, true, 3, 4, 4, 4, 4, 4>(a, slices, part, s)
+                         : go_mt<EPI_RESID, false, true, 3, 10, 8, 6, 4, 2>(a, slices, part, s);
     if (st) return st;
-    return slices == 4 ? finish<4>(part, a.h, chain.next_nw, chain.next_xn, nullptr, a.ss_out,
-                                   a.mrows, a.N, a.eps, s)
-                       : finish<8>(part, a.h, chain.next_nw, chain.next_xn, nullptr, a.ss_out,
-                                   a.mrows, a.N, a.eps, s);
+    return finish<4>(part, a.h, chain.next_nw, chain.next_xn, nullptr, a.ss_out, a.mrows, a.N,
+                     a.eps, s);
   }
   // x in the operand order: given by the caller's previous projection, or normed here
   uint16_t* xn = reinterpret_cast<uint16_t*>(part);

@@ -42,13 +42,13 @@ struct RowsChain {
 int launch_layout5(GemvArgs a, int epi, bool norm, int tn, int slices, const RowsChain& chain,
                    float* part, hipStream_t s);
 // K = 2560 behind a norm (F32 and BF16 with 2 tiles per workgroup, SWIGLU 3, ARGMAX 4 or
-// 6), one slice; RESID without a norm, 4 slices of 3 tiles (K = 4096, 9728) or 8 of 5
-// (9728): about one workgroup per CU at N = 2560.
+// 6), one slice; RESID without a norm, K = 4096 or 9728 in 4 slices of 3 tiles (216
+// workgroups at N = 2560; 8 slices of 5 tiles, 256 of them, write twice the sums: down at
+// 32 / 64 rows 14.6 / 18.4 against 14.0 / 17.2 us).
 inline bool rows_supported(int N, int K, int epi, bool norm, int tn, int slices) {
   if (epi == EPI_RESID)
-    return !norm && (N & 3) == 0 && N <= 8192 &&
-           ((slices == 4 && tn == 3 && (K == 4096 || K == 9728)) ||
-            (slices == 8 && tn == 5 && K == 9728));
+    return !norm && (N & 3) == 0 && N <= 8192 && slices == 4 && tn == 3 &&
+           (K == 4096 || K == 9728);
   if (!norm || K != 2560 || slices != 1) return false;
   if (epi == EPI_ARGMAX) return tn == 4 || tn == 6;
   return tn == (epi == EPI_SWIGLU ? 3 : 2);

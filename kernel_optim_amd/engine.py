@@ -234,12 +234,11 @@ def build_decode_gemvs(cfg, M, raw, deadline, tiled_fn=None, tune=True, log="", 
                      else [tile_weights(w, swiglu=name == "gu") for w in raw[name]])
         if tune and M > 16 and g.rows_cfgs():
             # From 17 rows on the better layout is clear: layout 5 for the layers, where o and
-            # gate/up gain more as a pair (one norm less) than the tuner sees (32 rows: 9.7 +
-            # 20.5 us against 10.5 + 24.3, down 15.1 against 19.5, qkv with its norm 12.0
-            # against 14.3), down in 8 slices above 32 rows (64 rows 19.2 against 20.0, 32
-            # rows 15.6 against 15.1); the LM head on layout 2 up to 32 rows (150 against 158
-            # us; 48 rows 285 against 191).
-            g.cfg = g.rows_cfgs()[0 if M > 32 else -1]
+            # gate/up gain more as a pair (one norm less) than the tuner sees (32 rows: 8.9 +
+            # 20.5 us against 10.5 + 24.3, down 14.0 against 19.5, qkv with its norm 12.0
+            # against 14.3); the LM head on layout 2 up to 32 rows (150 against 158 us; 48
+            # rows 285 against 191).
+            g.cfg = g.rows_cfgs()[0]
             if name == "lm" and M <= 32:
                 g.cfg = (2, 1, 2)
             _log(f"{log}gemv {name} M={M} cfg={g.cfg} (rule)")

@@ -111,9 +111,8 @@ class Gemv:
         """Layout 5's configurations of this projection, the better one at more than 32
         rows first (gemv_launch.h, rows_supported)."""
         if self.epi == EPI_RESID:
-            if self.norm or self.N % 4 or self.N > 8192:
-                return []
-            return {4096: [(5, 3, 4)], 9728: [(5, 5, 8), (5, 3, 4)]}.get(self.K, [])
+            ok = not self.norm and self.N % 4 == 0 and self.N <= 8192 and self.K in (4096, 9728)
+            return [(5, 3, 4)] if ok else []
         if not self.norm or self.K != 2560:
             return []
         return {EPI_SWIGLU: [(5, 3, 1)], EPI_ARGMAX: [(5, 6, 1), (5, 4, 1)]}.get(
