@@ -122,7 +122,8 @@ def _row_sums_exact(device, n):
 
 
 def _plain(t, dev, *shape):
-    return (t.dtype == BF16 and t.device == dev and tuple(t.shape) == shape
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == BF16
+            and t.device == dev and tuple(t.shape) == shape
             and t.is_contiguous() and t.data_ptr() % 16 == 0)
 
 
@@ -143,7 +144,8 @@ def _rows_served(cfg, embed, B, S, k_cache, v_cache, cos, sin):
             and cache(k_cache) and cache(v_cache) and k_cache.stride() == v_cache.stride()
             and _plain(cos, dev, cos.shape[0], d) and _plain(sin, dev, sin.shape[0], d)
             and min(cos.shape[0], sin.shape[0]) >= S and embed.dtype == BF16
-            and not torch.is_autocast_enabled() and _row_sums_exact(dev, H))
+            and not torch.is_autocast_enabled() and not torch.compiler.is_compiling()
+            and _row_sums_exact(dev, H))
 
 
 def _layer_served(cfg, lw, dev):
