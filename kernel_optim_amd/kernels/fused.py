@@ -99,8 +99,9 @@ class DecodeAttention:
     4x the per-wavefront share.
 
     A second launch merges the partials, as the reference does, where the units take
-    several rounds of the grid; with one round, or ``fused_combine``, the last unit of each (sequence, KV head) merges them in
-    the same launch instead, through an arrival counter. The partials and the
+    several rounds of the grid; with one round, or ``fused_combine``, the last unit of each
+    (sequence, KV head) merges them in the same launch instead, through an arrival counter
+    (a pair of a single unit writes its output itself). The partials and the
     counter travel through device-coherent stores, loads and atomics (no fence,
     no L2 write-back).
     """
