@@ -60,11 +60,11 @@ FUSE_OPROJ = os.environ.get("ENGINE_FUSE_OPROJ", "1") == "1"
 OPROJ_DELAY_NS = int(os.environ.get("ENGINE_OPROJ_DELAY_NS", "1000"))
 # keys per decode-attention unit (0: DecodeAttention's sizing rule)
 ATTN_UNIT = int(os.environ.get("ENGINE_ATTN_UNIT", "0"))
-# units per sequence of the one-token attention at B >= 3 (-1: one round of the
-# 256 CUs, 256 // (B * KV heads); 0: fixed units of ATTN_UNIT or the sizing rule)
+# units per sequence of the one-token attention at B >= 3 (-1: whole rounds of the
+# 256 CUs, attn_units_per_seq; 0: fixed units of ATTN_UNIT or the sizing rule)
 ATTN_SPLIT = int(os.environ.get("ENGINE_ATTN_SPLIT", "-1"))
-# decode-step graph: "auto" takes the fused-GEMV step up to FUSED_MAX_B sequences
-# and the hipBLASLt step above; "timed" captures both up to FUSED_MAX_TIMED and
+# decode-step graph: "auto" takes the fused-GEMV step up to FUSED_MAX_B sequences (64
+# where layout 5 serves the widths) and the hipBLASLt step above; "timed" captures both up to FUSED_MAX_TIMED and
 # keeps the faster, as the reference does (engine.py:197-208); "fused" or
 # "hipblaslt" takes one
 DECODE_GRAPH = os.environ.get("ENGINE_DECODE_GRAPH", "auto")
