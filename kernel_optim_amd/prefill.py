@@ -23,7 +23,9 @@ The prompt's K (normed + roped) and V go to cache slots 0..S-1.
 """
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from .kernels.fused import prefill_norm, prefill_qkv, silu_mul2
 
@@ -121,6 +123,24 @@ def _row_sums_exact(device, n):
     return _ROW_SUMS[key]
 
 
+def _observed():
+    """Whether something records, rewrites or differentiates the torch operations of this
+    call: a trace (jit, dynamo, make_fx), a dispatch or function mode, a functorch transform
+    (vmap, functionalize, jvp) or a forward-mode level. The row kernels work by address and
+    would be missing from what it sees. A default device (DeviceContext) rewrites nothing here."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._len_torch_dispatch_stack() > 0
+            or torch._ops._len_torch_dispatch_stack_pre_dispatch() > 0
+            or any(not isinstance(m, DeviceContext)
+                   for m in torch.overrides._get_current_function_mode_stack())
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or forward_ad._current_level >= 0)
+
+
+def _on_gpu(dev):
+    return dev.type == "cuda" and dev.index in (None, torch.cuda.current_device())
+
+
 def _plain(t, dev, *shape):
     return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == BF16
             and t.device == dev and tuple(t.shape) == shape
@@ -128,9 +148,11 @@ def _plain(t, dev, *shape):
 
 
 def _rows_served(cfg, embed, B, S, k_cache, v_cache, cos, sin):
-    """Whether the row kernels serve this call: bf16 tensors on the current GPU in the
-    engine's layouts, heads of 128, and rows whose mean of squares they add in torch's
-    order (which changes below 8 rows, below 256 values and past 8064)."""
+    """Whether the row kernels serve this call: made eagerly (_observed), with bf16 tensors
+    on the current GPU in the engine's layouts, heads of 128, and rows whose mean of squares
+    they add in torch's order (which changes below 8 rows, below 256 values and past 8064)."""
+    if _observed():
+        return False
     H, d, dev = cfg.hidden, cfg.head_dim, k_cache.device
 
     def cache(t):
@@ -139,13 +161,12 @@ def _rows_served(cfg, embed, B, S, k_cache, v_cache, cos, sin):
                 and t.stride(4) == 1 and t.stride(3) == d and t.data_ptr() % 16 == 0
                 and all(t.stride(i) % 8 == 0 for i in range(3)))
 
-    return (dev.type == "cuda" and B * S >= 8 and 256 <= H <= 8064 and H % 8 == 0 and d == 128
-            and cfg.inter % 8 == 0 and dev.index in (None, torch.cuda.current_device())
+    return (_on_gpu(dev) and B * S >= 8 and 256 <= H <= 8064 and H % 8 == 0 and d == 128
+            and cfg.inter % 8 == 0
             and cache(k_cache) and cache(v_cache) and k_cache.stride() == v_cache.stride()
             and _plain(cos, dev, cos.shape[0], d) and _plain(sin, dev, sin.shape[0], d)
             and min(cos.shape[0], sin.shape[0]) >= S and embed.dtype == BF16
-            and not torch.is_autocast_enabled() and not torch.compiler.is_compiling()
-            and _row_sums_exact(dev, H))
+            and not torch.is_autocast_enabled() and _row_sums_exact(dev, H))
 
 
 def _layer_served(cfg, lw, dev):

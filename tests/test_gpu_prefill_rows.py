@@ -102,3 +102,22 @@ def test_prefill_row_kernels_keep_the_torch_path_bits(dev, monkeypatch, B, S, kw
     monkeypatch.setattr(P, "_rows_served", lambda *a: False)
     for a, b in zip(got, once()):
         assert torch.equal(a, b)
+
+
+def test_a_traced_prefill_replays_the_forward(dev):
+    """torch.jit.trace records torch operations only, so it gets nothing else: a replay on
+    other tokens has the eager call's bits."""
+    cfg = Qwen3Config(layers=2, vocab=64)
+    w = random_weights(cfg, seed=3, device=dev)
+    cos, sin = _randn(None, 40, 128), _randn(None, 40, 128)
+
+    def f(prompt, kc, vc):
+        kc, vc = kc.clone(), vc.clone()
+        return (*P.prefill(cfg, w, prompt, kc, vc, cos, sin), kc, vc)
+
+    kc = torch.zeros(2, 2, cfg.nkv, 40, 128, dtype=BF, device=dev)
+    one, other = (torch.randint(0, cfg.vocab, (2, 33), device=dev) for _ in range(2))
+    f(one, kc, kc)   # the probes of this device and width, outside the trace
+    traced = torch.jit.trace(f, (one, kc, kc), check_trace=False)
+    for a, b in zip(traced(other, kc, kc), f(other, kc, kc)):
+        assert torch.equal(a, b)
