@@ -141,10 +141,15 @@ def _on_gpu(dev):
     return dev.type == "cuda" and dev.index in (None, torch.cuda.current_device())
 
 
+def _is_plain(t):
+    """No subclass, whose operations may be its own: a layer with one, and the layers that
+    read what it returns, keep the torch operations."""
+    return type(t) in (torch.Tensor, torch.nn.Parameter)
+
+
 def _plain(t, dev, *shape):
-    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == BF16
-            and t.device == dev and tuple(t.shape) == shape
-            and t.is_contiguous() and t.data_ptr() % 16 == 0)
+    return (_is_plain(t) and t.dtype == BF16 and t.device == dev
+            and tuple(t.shape) == shape and t.is_contiguous() and t.data_ptr() % 16 == 0)
 
 
 def _rows_served(cfg, embed, B, S, k_cache, v_cache, cos, sin):
@@ -156,7 +161,8 @@ def _rows_served(cfg, embed, B, S, k_cache, v_cache, cos, sin):
     H, d, dev = cfg.hidden, cfg.head_dim, k_cache.device
 
     def cache(t):
-        return (t.dtype == BF16 and t.device == dev and t.dim() == 5 and t.shape[1] == B
+        return (_is_plain(t) and t.dtype == BF16 and t.device == dev and t.dim() == 5
+                and t.shape[1] == B
                 and t.shape[2] == cfg.nkv and t.shape[3] >= S and t.shape[4] == d
                 and t.stride(4) == 1 and t.stride(3) == d and t.data_ptr() % 16 == 0
                 and all(t.stride(i) % 8 == 0 for i in range(3)))
@@ -165,15 +171,15 @@ def _rows_served(cfg, embed, B, S, k_cache, v_cache, cos, sin):
             and cfg.inter % 8 == 0
             and cache(k_cache) and cache(v_cache) and k_cache.stride() == v_cache.stride()
             and _plain(cos, dev, cos.shape[0], d) and _plain(sin, dev, sin.shape[0], d)
-            and min(cos.shape[0], sin.shape[0]) >= S and embed.dtype == BF16
+            and min(cos.shape[0], sin.shape[0]) >= S and _is_plain(embed) and embed.dtype == BF16
             and not torch.is_autocast_enabled() and _row_sums_exact(dev, H))
 
 
-def _layer_served(cfg, lw, dev):
-    H, d = cfg.hidden, cfg.head_dim
-    return (_plain(lw["w_in"], dev, H) and _plain(lw["w_post"], dev, H)
+def _layer_served(cfg, lw, x):
+    H, d, dev = cfg.hidden, cfg.head_dim, x.device
+    return (_plain(x, dev, *x.shape) and _plain(lw["w_in"], dev, H) and _plain(lw["w_post"], dev, H)
             and _plain(lw["q_norm"], dev, d) and _plain(lw["k_norm"], dev, d)
-            and lw["qkv"].dtype == lw["o"].dtype == lw["gu"].dtype == lw["down"].dtype == BF16)
+            and all(_is_plain(lw[n]) and lw[n].dtype == BF16 for n in ("qkv", "o", "gu", "down")))
 
 
 def _layer_rows(cfg, lw, x, delta, h, kc, vc, cos, sin, exact_gqa):
@@ -232,11 +238,12 @@ def prefill(cfg, w, prompt, k_cache, v_cache, cos, sin):
     B, S = prompt.shape
     exact_gqa = gqa_exact(prompt.device)
     x = F.embedding(prompt, w["embed"])
-    rows = _rows_served(cfg, w["embed"], B, S, k_cache, v_cache, cos, sin)
+    rows = (_is_plain(prompt)
+            and _rows_served(cfg, w["embed"], B, S, k_cache, v_cache, cos, sin))
     h = torch.empty_like(x) if rows else None
     delta = None   # the last layer's output where it is not yet in x
     for i, lw in enumerate(w["layers"]):
-        if rows and _layer_served(cfg, lw, x.device):
+        if rows and _layer_served(cfg, lw, x):
             delta = _layer_rows(cfg, lw, x, delta, h, k_cache[i], v_cache[i], cos, sin, exact_gqa)
             continue
         if delta is not None:

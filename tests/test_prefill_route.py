@@ -110,3 +110,35 @@ def test_forward_mode_keeps_the_tangents(rows):
         w["final_norm"] = fad.make_dual(w["final_norm"], torch.ones_like(w["final_norm"]))
         logits = P.prefill(CFG, w, prompt, kc, vc, cos, sin)[1]
         assert fad.unpack_dual(logits).tangent is not None
+
+
+class Logged(torch.Tensor):
+    """A subclass whose operations return it, as a wrapper or a distributed tensor does."""
+
+
+@pytest.mark.parametrize("name", ["prompt", "k_cache", "v_cache", "cos", "sin", "embed", "w_in",
+                                  "w_post", "q_norm", "k_norm", "qkv", "o", "gu", "down"])
+def test_tensor_subclasses_keep_the_torch_operations(rows, name):
+    """In any argument, and in the first layer (whose output then is one too)."""
+    args = list(_inputs())
+    want = _torch_route(args)
+    at = ("w", "prompt", "k_cache", "v_cache", "cos", "sin")
+    if name in at:
+        args[at.index(name)] = args[at.index(name)].as_subclass(Logged)
+    elif name == "embed":
+        args[0]["embed"] = args[0]["embed"].as_subclass(Logged)
+    else:
+        args[0]["layers"][0][name] = args[0]["layers"][0][name].as_subclass(Logged)
+    if name in at or name == "embed":
+        _same([t.as_subclass(torch.Tensor) for t in _call(*args)], want)
+        return
+    reached = []
+    plain = P._layer_torch
+    P._layer_torch = lambda *a: reached.append(plain(*a)) or reached[-1]
+    try:
+        # the norms' results are subclasses, but the products of plain weights are too: the
+        # second layer's input decides
+        _same([t.as_subclass(torch.Tensor) for t in _call(*args)], want)
+    finally:
+        P._layer_torch = plain
+    assert len(reached) == 2 and type(reached[0]) is Logged
