@@ -99,10 +99,10 @@ class DecodeAttention:
     4x the per-wavefront share.
 
     A second launch merges the partials, as the reference does, where the units take
-    several rounds of the grid; with one round, or ``fused_combine``, the last unit of each
-    (sequence, KV head) merges them in the same launch instead, through an arrival counter
-    (a pair of a single unit writes its output itself). The partials and the
-    counter travel through device-coherent stores, loads and atomics (no fence,
+    several rounds of the grid or more than 24 meet in a (sequence, KV head) pair; else, or
+    with ``fused_combine``, the last unit of each pair merges them in the same launch
+    instead, through an arrival counter (a pair of a single unit writes its output itself).
+    The partials and the counter travel through device-coherent stores, loads and atomics (no fence,
     no L2 write-back).
     """
 
@@ -151,11 +151,15 @@ class DecodeAttention:
         self.counters = words[n_sync + 4:] if fused_combine else None
         # The two-launch form of one query token whose units are one round of the grid
         # merges in its one launch too, on these counters: the bits of two launches (B = 1,
-        # 512 keys: 8.9 -> 7.2 us; 4 x 2048 15.1 -> 13.1; 16 x 8192 83.6 -> 81.4).
+        # 512 keys: 8.9 -> 7.2 us; 4 x 2048 15.1 -> 13.1; 16 x 8192 83.6 -> 81.4), up to 24
+        # units a pair: its last workgroup merges them 32 slots at a time and a row per
+        # wavefront, where the second launch has a wavefront for every row of the grid (one
+        # sequence, 16 / 22 / 25 / 32 / 64 units of 64: 8.6 / 9.4 / 9.8 / 10.7 / 15.8 us
+        # against 9.3 / 9.6 / 9.7 / 10.0 / 12.5).
         # Several rounds stay with two launches (ragged B = 64 5,887 against 5,771 GB/s).
         one_round = B * nkv * self.max_units * self.waves_per_unit <= self.grid_waves
         self._own_counters = (words[n_sync + 4:] if T == 1 and not fused_combine and one_round
-                              else None)
+                              and self.max_units <= 24 else None)
         self.oproj_delay_ns = 1000
         # polls of a pair's done flag before a decode_qkv_oproj wait gives up and
         # sets err (-1: the library's bound; 0: give up at once, for tests)
@@ -164,6 +168,11 @@ class DecodeAttention:
         self._q_shape = torch.Size((B * T, nq * d))
         self._kv_shape = torch.Size((B, nkv, cap, d))
         self._len_shape = torch.Size((B,))
+
+    @property
+    def one_launch(self):
+        """Whether __call__ and with_lengths merge the partials in their one launch."""
+        return self.counters is not None or self._own_counters is not None
 
     def _check_kv(self, k_cache, v_cache, lens):
         B, nkv, d, cap = self.B, self.nkv, self.d, self.cap
