@@ -113,7 +113,9 @@ int ko_decode_attn_token_rows(const void* q, const void* k_cache, const void* v_
  * given, B <= 64, unit % 64 == 0): each sequence's pos[b] + 1 keys are cut
  * into at most U units of equal size, rounded up to a multiple of 64 and at
  * least `unit` keys, from its length at this step, or left whole below 2.5
- * `unit` keys (max_units * unit >= cap still sizes the partials). */
+ * `unit` keys, and below 4 `unit` cut into one round of the 256 CUs, 256 / (B *
+ * nkv) units, where that is 2 or more and less than U (max_units * unit >= cap
+ * still sizes the partials). */
 int ko_decode_attn_qkv(const void* qkv, const void* q_w, const void* k_w, const void* cos,
                        const void* sin, int max_pos, const int* pos, void* k_cache,
                        void* v_cache, int cap, long long cache_b_stride,

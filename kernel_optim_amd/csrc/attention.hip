@@ -799,7 +799,12 @@ int ko_decode_attn_qkv(const void* qkv, const void* q_w, const void* k_w, const 
   a.counters = counters;
   a.out = static_cast<uint16_t*>(out);
   a.rope = static_cast<const uint16_t*>(rope);
-  a.usplit = units_per_seq;
+  // More units than one round of the 256 CUs pay from 4 smallest units on, where a round has
+  // two or more per sequence (12 sequences of 320 / 450 keys, up to 5 units of 128: 12.1 / 12.9
+  // us in those, 11.1 / 12.5 in 2 units; 800 keys 15.7 against 16.6).
+  const int most = units_per_seq < 0x7fff ? units_per_seq : 0x7fff;
+  const int round = (long long)B * nkv <= 128 ? 256 / (B * nkv) : 1;
+  a.usplit = most | (round >= 2 && round < most ? round : most) << 16;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (counters) return launch1<true, true>(a, grid_waves, s);
   st = launch1<true, false>(a, grid_waves, s);

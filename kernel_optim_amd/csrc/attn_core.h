@@ -55,7 +55,8 @@ struct AttnArgs {
   int B, nkv, unit, max_units;
   // One-token kernel, B <= 64, fused merge: cut each sequence's keys into at
   // most usplit units of equal size (a multiple of 64, at least `unit`) from
-  // its current length, instead of fixed units of `unit` keys (0: fixed).
+  // its current length, instead of fixed units of `unit` keys (0: fixed). Two counts in
+  // one register: the low 16 bits, and above them the one for less than 4 `unit`.
   int usplit;
   // Query tokens per sequence in the q / out / partial row layout (T of the
   // call), and the first token this launch serves: calls of more than 4
@@ -84,10 +85,12 @@ __device__ __forceinline__ int nunits(int len, int unit) {
 // length cut into usplit parts, rounded up to a multiple of 64, at least `unit`; a
 // sequence of less than 2.5 `unit` is left whole (it then writes its output itself,
 // which is worth more than the second workgroup: 12 sequences of 100 keys 8.6 us in
-// units of 64, 7.3 whole; 40 of 640 keys 32.6 in units of 320, 28.3 whole).
+// units of 64, 7.3 whole; 40 of 640 keys 32.6 in units of 320, 28.3 whole), and one of
+// less than 4 `unit` cut into one round of the CUs (attention.hip, ko_decode_attn_qkv).
 __device__ __forceinline__ int unit_for(int len, int unit, int usplit) {
   if (usplit <= 0 || len <= 0) return unit;
-  const int parts = 2 * len < 5 * unit ? 1 : usplit;
+  const int half = len < 4 * unit ? 16 : 0;
+  const int parts = 2 * len < 5 * unit ? 1 : (usplit >> half) & 0xffff;
   const int u = ((len + parts - 1) / parts + 63) & ~63;
   return u > unit ? u : unit;
 }

@@ -122,8 +122,8 @@ class DecodeAttention:
         # units_per_seq = U > 0: decode_qkv cuts each sequence's keys into at most U
         # equal units (multiples of 64 keys, at least `unit`) from its length at
         # each step, so a batch of equal lengths fills whole rounds of the grid
-        # whatever the position; less than 2.5 `unit` keys stay whole
-        # (ko_decode_attn_qkv)
+        # whatever the position; less than 2.5 `unit` keys stay whole, less than 4 take
+        # one round of the CUs (ko_decode_attn_qkv)
         self.units_per_seq = int(units_per_seq)
         if self.units_per_seq:
             _need(self.units_per_seq > 0 and T == 1 and not self.token_rows and fused_combine

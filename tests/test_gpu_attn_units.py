@@ -69,6 +69,34 @@ def test_per_sequence_units(dev, split, unit):
     torch.testing.assert_close(out.cpu().double(), want, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("B,split,lens,parts", [
+    (12, 5, [1, 319, 320, 321, 400, 511, 512, 513, 640, 641, 800, 1500],
+     [1, 1, 2, 2, 2, 2, 4, 5, 5, 4, 5, 5]),
+    (4, 8, [159, 160, 255, 256], [1, 3, 4, 4]),          # one round: 8 units, of at least 64
+    (17, 3, [799, 800, 1279, 1280] * 4 + [1], [1, 3, 3, 3] * 4 + [1])])   # one unit a round
+def test_units_that_a_sequence_is_cut_into(dev, B, split, lens, parts):
+    """Counted by the partials that it leaves (a whole sequence leaves none). More units than
+    one round of the CUs are taken from 4 smallest units on."""
+    cap = -(-max(lens) // 16) * 16
+    q, k, v = _case(dev, B, cap, split)
+    g = torch.Generator(device=dev).manual_seed(7)
+    qkv = torch.randn(B, 48 * 128, device=dev, generator=g).to(BF)
+    ones = torch.ones(128, dtype=BF, device=dev)
+    cos, sin = torch.ones(cap, 128, dtype=BF, device=dev), torch.zeros(cap, 128, dtype=BF, device=dev)
+    pos = torch.tensor(lens, dtype=torch.int32, device=dev) - 1
+    op = DecodeAttention(B, 1, cap, 32, 8, 128, dev, fused_combine=True, units_per_seq=split)
+    op.ml.fill_(float("nan"))
+    out = torch.zeros_like(q)
+    op.decode_qkv(qkv, ones, ones, cos, sin, pos, k, v, out, 1e-6)
+    n = (~op.ml.view(B, 32, op.max_units, 2)[..., 0].isnan()).sum(-1)
+    assert torch.equal(n, n[:, :1].expand(-1, 32))
+    assert n[:, 0].tolist() == [p if p > 1 else 0 for p in parts]
+    from kernel_optim_amd.prefill import rmsnorm
+    qn = rmsnorm(qkv[:, :32 * 128].view(B, 32, 128), ones, 1e-6).view(B, -1)
+    want = A.decode_attention(qn.cpu(), k.cpu(), v.cpu(), lens)
+    torch.testing.assert_close(out.cpu().double(), want, atol=2e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("B,lens", [(1, [0]), (70, [0, 5] * 35)])
 def test_sequences_without_keys_give_zeros(dev, B, lens):
     """One sequence, and more than 64 (whose lengths are read in chunks)."""
