@@ -584,8 +584,9 @@ def bench_attention(args):
     pos = torch.full((B,), CTX - 1, dtype=torch.int32, device=dev)
     out = torch.empty_like(q)
     # the reference's two-launch form (partials, then a combine launch)
-    att = DecodeAttention(B, 1, CTX, NQ, NKV, D, dev)
-    # the form the engine runs: partials and the LSE merge in one launch
+    att = DecodeAttention(B, 1, CTX, NQ, NKV, D, dev, two_launches=True)
+    # the form the engine runs, and the op's own choice at this size: partials and the LSE
+    # merge in one launch
     att2 = DecodeAttention(B, 1, CTX, NQ, NKV, D, dev, fused_combine=True)
     print(f"[bench] attention B={B} ctx={CTX} unit={att.unit} units={att.max_units * B * NKV} "
           f"grid_waves={att.grid_waves}", file=sys.stderr, flush=True)

@@ -99,8 +99,8 @@ class DecodeAttention:
     4x the per-wavefront share.
 
     A second launch merges the partials, as the reference does, where the units take
-    several rounds of the grid or more than 24 meet in a (sequence, KV head) pair; else, or
-    with ``fused_combine``, the last unit of each pair merges them in the same launch
+    several rounds of the grid or more than 24 meet in a (sequence, KV head) pair, or
+    always with ``two_launches``; else, or with ``fused_combine``, the last unit of each pair merges them in the same launch
     instead, through an arrival counter (a pair of a single unit writes its output itself).
     The partials and the counter travel through device-coherent stores, loads and atomics (no fence,
     no L2 write-back).
@@ -109,12 +109,13 @@ class DecodeAttention:
     MAX_T = 8
 
     def __init__(self, B, T, cap, nq, nkv, d, device, target_ctas=2048, unit=None,
-                 fused_combine=False, token_rows=False, units_per_seq=0):
+                 fused_combine=False, token_rows=False, units_per_seq=0, two_launches=False):
         _need(d == 128, "head_dim must be 128")
         _need(nq == 4 * nkv, "the kernel serves GQA groups of 4 query heads per KV head")
         _need(1 <= T <= self.MAX_T, f"T must be in 1..{self.MAX_T}")
         _need(not token_rows or (T >= 2 and fused_combine),
               "token_rows serves T >= 2 with the fused combine")
+        _need(not (two_launches and fused_combine), "two_launches excludes fused_combine")
         self.B, self.T, self.cap, self.nq, self.nkv, self.d = B, T, cap, nq, nkv, d
         # token_rows: the T tokens of a sequence run as T rows of the one-token
         # kernel (ko_decode_attn_token_rows), each with its own causal length
@@ -158,8 +159,9 @@ class DecodeAttention:
         # against 9.3 / 9.6 / 9.7 / 10.0 / 12.5).
         # Several rounds stay with two launches (ragged B = 64 5,887 against 5,771 GB/s).
         one_round = B * nkv * self.max_units * self.waves_per_unit <= self.grid_waves
-        self._own_counters = (words[n_sync + 4:] if T == 1 and not fused_combine and one_round
-                              and self.max_units <= 24 else None)
+        own = (T == 1 and one_round and self.max_units <= 24
+               and not (fused_combine or two_launches))
+        self._own_counters = words[n_sync + 4:] if own else None
         self.oproj_delay_ns = 1000
         # polls of a pair's done flag before a decode_qkv_oproj wait gives up and
         # sets err (-1: the library's bound; 0: give up at once, for tests)

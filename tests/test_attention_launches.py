@@ -20,3 +20,14 @@ def test_one_launch_only_where_few_units_meet_in_a_pair(B, cap, units, one):
     assert op.max_units == units
     assert op.one_launch == one and op.counters is None
     assert _op(B, cap, fused_combine=True).one_launch
+
+
+def test_two_launches_can_be_asked_for():
+    """The reference's form, which a comparison of the two has to name."""
+    for B, cap in ((16, 8192), (1, 512), (64, 16384)):
+        assert not _op(B, cap, two_launches=True).one_launch
+    with pytest.raises(ValueError, match="two_launches"):
+        _op(1, 512, two_launches=True, fused_combine=True)
+    with pytest.raises(ValueError, match="two_launches"):
+        DecodeAttention(2, 3, 512, 32, 8, 128, "cpu", two_launches=True, fused_combine=True,
+                        token_rows=True)

@@ -126,7 +126,8 @@ def test_config2_b16_ctx8192(dev):
     q, k, v = _inputs(B, 1, cap, dev)
     pos = torch.full((B,), cap - 1, dtype=torch.int32, device=dev)
     out = torch.empty_like(q)
-    att = fused.DecodeAttention(B, 1, cap, 32, 8, 128, dev)
+    att = fused.DecodeAttention(B, 1, cap, 32, 8, 128, dev, two_launches=True)
+    assert not att.one_launch
     att(q, k, v, pos, out)
     torch.cuda.synchronize()
     ref = _gpu_ref_fp32(q, k, v, [cap] * B)
@@ -134,8 +135,8 @@ def test_config2_b16_ctx8192(dev):
     sel = [0, 5, 10, 15]
     want = A.decode_attention(q.view(B, -1)[sel].cpu(), k[sel].cpu(), v[sel].cpu(), [cap] * 4)
     torch.testing.assert_close(out.view(B, -1)[sel].cpu().double(), want, **TOL)
-    # the same op with the merge in the partial launch (as the engine and the
-    # benchmark run it): bit-identical, on repeated launches
+    # the same op with the merge in the partial launch (as the engine runs it):
+    # bit-identical, on repeated launches
     attf = fused.DecodeAttention(B, 1, cap, 32, 8, 128, dev, fused_combine=True)
     for _ in range(3):
         outf = torch.zeros_like(q)
@@ -177,7 +178,9 @@ def test_long_context_65536(dev, fused_combine):
     k[1, :, 40001:] = float("nan")
     v[1, :, 40001:] = float("nan")
     out = torch.empty_like(q)
-    att = fused.DecodeAttention(B, 1, cap, 32, 8, 128, dev, fused_combine=fused_combine)
+    att = fused.DecodeAttention(B, 1, cap, 32, 8, 128, dev, fused_combine=fused_combine,
+                                two_launches=not fused_combine)
+    assert att.one_launch == fused_combine
     att.with_lengths(q, k, v, lens.to(dev), out)
     torch.cuda.synchronize()
     assert torch.isfinite(out.float()).all()
@@ -201,7 +204,9 @@ def test_more_than_64_sequences(dev, fused_combine):
         k[b, :, int(lens[b]):] = float("nan")
         v[b, :, int(lens[b]):] = float("nan")
     out = torch.empty_like(q)
-    att = fused.DecodeAttention(B, 1, cap, 32, 8, 128, dev, fused_combine=fused_combine)
+    att = fused.DecodeAttention(B, 1, cap, 32, 8, 128, dev, fused_combine=fused_combine,
+                                two_launches=not fused_combine)
+    assert att.one_launch == fused_combine
     att.with_lengths(q, k, v, lens.to(dev), out)
     torch.cuda.synchronize()
     assert torch.isfinite(out.float()).all()
@@ -273,7 +278,9 @@ def test_two_launch_and_fused_combine_agree(dev, fused):
     B, cap = 5, 700
     q, k, v = _inputs(B, 1, cap, dev, seeds=(19, 20, 21))
     pos = torch.tensor([699, 0, 63, 64, 350], dtype=torch.int32, device=dev)
-    att = fused_mod.DecodeAttention(B, 1, cap, 32, 8, 128, dev, unit=64, fused_combine=fused)
+    att = fused_mod.DecodeAttention(B, 1, cap, 32, 8, 128, dev, unit=64, fused_combine=fused,
+                                    two_launches=not fused)
+    assert att.one_launch == fused
     out = torch.empty_like(q)
     for _ in range(3):  # counters must re-arm between launches
         att(q, k, v, pos, out)

@@ -26,11 +26,10 @@ def test_a_pair_of_one_unit_keeps_the_merged_bits(dev, unit):
     q, k, v = _case(dev, len(lens), cap, unit)
     n = torch.tensor(lens, dtype=torch.int32, device=dev)
     outs = []
-    for fused in (True, False, None):   # one launch asked for, two launches, one by the op's rule
-        op = DecodeAttention(len(lens), 1, cap, 32, 8, 128, dev, unit=unit,
-                             fused_combine=bool(fused))
-        if fused is False:
-            op._own_counters = None
+    # one launch asked for, two launches, one by the op's rule
+    for kw in (dict(fused_combine=True), dict(two_launches=True), {}):
+        op = DecodeAttention(len(lens), 1, cap, 32, 8, 128, dev, unit=unit, **kw)
+        assert op.one_launch == ("two_launches" not in kw)
         out = torch.full_like(q, float("nan"))
         for _ in range(2):   # the counters are left at zero
             op.with_lengths(q, k, v, n, out)
@@ -103,10 +102,9 @@ def test_sequences_without_keys_give_zeros(dev, B, lens):
     q, k, v = _case(dev, B, 16, B)
     n = torch.tensor(lens, dtype=torch.int32, device=dev)
     outs = []
-    for own in (True, False):
-        op = DecodeAttention(B, 1, 16, 32, 8, 128, dev, unit=16)
-        assert op._own_counters is not None
-        op._own_counters = op._own_counters if own else None
+    for two in (False, True):
+        op = DecodeAttention(B, 1, 16, 32, 8, 128, dev, unit=16, two_launches=two)
+        assert op.one_launch != two
         out = torch.full_like(q, float("nan"))
         op.with_lengths(q, k, v, n, out)
         outs.append(out)

@@ -45,7 +45,7 @@ def _noalloc(att, q, k, v, pos, out, max_units=None):
 def test_noalloc_matches_the_scratch_entry_point(dev):
     for B, cap, lens, seed in ((16, 8192, [8192] * 16, 1), (3, 700, [700, 1, 333], 2)):
         q, k, v, pos = _case(dev, B, cap, lens, seed)
-        att = DecodeAttention(B, 1, cap, NQ, NKV, D, dev)   # two launches, own scratch
+        att = DecodeAttention(B, 1, cap, NQ, NKV, D, dev, two_launches=True)   # own scratch
         want = torch.empty_like(q)
         att(q, k, v, pos, want)
         got = torch.full_like(q, float("nan"))
@@ -57,7 +57,7 @@ def test_noalloc_matches_the_scratch_entry_point(dev):
 def test_noalloc_refuses_partials_beyond_its_array(dev):
     B, cap = 2, 4096
     q, k, v, pos = _case(dev, B, cap, [4096, 100], 3)
-    att = DecodeAttention(B, 1, cap, NQ, NKV, D, dev)
+    att = DecodeAttention(B, 1, cap, NQ, NKV, D, dev, two_launches=True)
     out = torch.zeros_like(q)
     # 2 x 32 rows x 600 units x 130 floats > 4 Mi floats: refused, nothing launched
     assert _noalloc(att, q, k, v, pos, out, max_units=600) == KO_ERANGE
@@ -87,7 +87,7 @@ q = torch.randn(B, NQ * D, device=dev, generator=g).to(torch.bfloat16)
 k = torch.randn(B, NKV, cap, D, device=dev, generator=g).to(torch.bfloat16)
 v = torch.randn(B, NKV, cap, D, device=dev, generator=g).to(torch.bfloat16)
 pos = torch.tensor([l - 1 for l in lens], dtype=torch.int32, device=dev)
-att = DecodeAttention(B, 1, cap, NQ, NKV, D, dev)  # no library launch yet
+att = DecodeAttention(B, 1, cap, NQ, NKV, D, dev, two_launches=True)  # no library launch yet
 out = torch.full_like(q, float("nan"))
 torch.cuda.synchronize()
 print("capturing the first ko_decode_attn_noalloc call", flush=True)
