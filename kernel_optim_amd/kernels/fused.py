@@ -159,8 +159,13 @@ class DecodeAttention:
         # against 9.3 / 9.6 / 9.7 / 10.0 / 12.5).
         # Several rounds stay with two launches (ragged B = 64 5,887 against 5,771 GB/s).
         one_round = B * nkv * self.max_units * self.waves_per_unit <= self.grid_waves
-        own = (T == 1 and one_round and self.max_units <= 24
+        # The counters must be zero for the stream of any first call: the constructor waits
+        # for their fill, and under capture, where it cannot, the two launches stay.
+        capturing = words.is_cuda and torch.cuda.is_current_stream_capturing()
+        own = (T == 1 and one_round and self.max_units <= 24 and not capturing
                and not (fused_combine or two_launches))
+        if own and words.is_cuda:
+            torch.cuda.current_stream(words.device).synchronize()
         self._own_counters = words[n_sync + 4:] if own else None
         self.oproj_delay_ns = 1000
         # polls of a pair's done flag before a decode_qkv_oproj wait gives up and

@@ -126,3 +126,47 @@ def test_bad_arguments_are_named(dev):
     for text, args in bad:
         with pytest.raises(ValueError, match=text):
             op.with_lengths(*args)
+
+
+def test_first_call_on_another_stream_than_the_objects(dev):
+    """The arrival counters are zero for every stream: the constructor waits for the fill,
+    here behind work on its own stream and over memory that held other words."""
+    q, k, v = _case(dev, 2, 512, 3)
+    n = torch.tensor([512, 300], dtype=torch.int32, device=dev)
+    want = A.decode_attention(q.cpu(), k.cpu(), v.cpu(), [512, 300])
+    out = torch.full_like(q, float("nan"))
+    torch.cuda.synchronize()
+    mine, other = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(mine):
+        size = DecodeAttention(2, 1, 512, 32, 8, 128, dev).sync.untyped_storage().nbytes()
+        old = torch.full((size // 4,), 7, dtype=torch.int32, device=dev)
+        del old
+        torch.cuda._sleep(20_000_000)
+        op = DecodeAttention(2, 1, 512, 32, 8, 128, dev)
+    assert op.one_launch
+    with torch.cuda.stream(other):
+        op.with_lengths(q, k, v, n, out)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(out.cpu().double(), want, atol=2e-2, rtol=2e-2)
+
+
+def test_an_object_made_under_capture_takes_two_launches(dev):
+    """Its counters would be zeroed by the replays only."""
+    q, k, v = _case(dev, 2, 512, 4)
+    n = torch.tensor([512, 300], dtype=torch.int32, device=dev)
+    want = A.decode_attention(q.cpu(), k.cpu(), v.cpu(), [512, 300])
+    out, eager = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    DecodeAttention(2, 1, 512, 32, 8, 128, dev, two_launches=True).with_lengths(q, k, v, n, out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        op = DecodeAttention(2, 1, 512, 32, 8, 128, dev)
+        op.with_lengths(q, k, v, n, out)
+    assert not op.one_launch
+    op.with_lengths(q, k, v, n, eager)   # before any replay
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+    torch.testing.assert_close(out.cpu().double(), want, atol=2e-2, rtol=2e-2)
