@@ -64,9 +64,9 @@ ATTN_UNIT = int(os.environ.get("ENGINE_ATTN_UNIT", "0"))
 # 256 CUs, attn_units_per_seq; 0: fixed units of ATTN_UNIT or the sizing rule)
 ATTN_SPLIT = int(os.environ.get("ENGINE_ATTN_SPLIT", "-1"))
 # decode-step graph: "auto" takes the fused-GEMV step up to FUSED_MAX_B sequences (64
-# where layout 5 serves the widths) and the hipBLASLt step above; "timed" captures both up to FUSED_MAX_TIMED and
-# keeps the faster, as the reference does (engine.py:197-208); "fused" or
-# "hipblaslt" takes one
+# where layout 5 serves the widths: auto_graph) and the hipBLASLt step above; "timed"
+# captures both up to FUSED_MAX_TIMED and keeps the faster, as the reference does
+# (engine.py:197-208); "fused" or "hipblaslt" takes one
 DECODE_GRAPH = os.environ.get("ENGINE_DECODE_GRAPH", "auto")
 # The fused GEMVs of any width read each weight once for up to 32 rows (B = 32: 8,619
 # tok/s against 7,544 on hipBLASLt); at 33..64 rows only layout 5 does, so "auto" takes
@@ -202,6 +202,15 @@ def rows_served(cfg):
         Gemv(64, H, cfg.nq * cfg.head_dim, EPI_RESID, norm=False, eps=e),
         Gemv(64, cfg.inter, H, EPI_SWIGLU, norm=True, eps=e),
         Gemv(64, H, cfg.inter, EPI_RESID, norm=False, eps=e)))
+
+
+def auto_graph(cfg, B):
+    """The decode graph of ``auto`` for B sequences: the fused GEMVs up to FUSED_MAX_B, and up
+    to ROWS_MAX where layout 5 serves the widths and build_decode_gemvs takes it (with tuning
+    off it keeps the row-major defaults, which at 33..64 rows read the weights four times:
+    a qkv projection 176 against 15 us)."""
+    rows = TUNE and rows_served(cfg)
+    return "fused" if B <= (ROWS_MAX if rows else FUSED_MAX_B) else "hipblaslt"
 
 
 def build_decode_gemvs(cfg, M, raw, deadline, tiled_fn=None, tune=True, log="", chain=False):
@@ -399,8 +408,7 @@ class Engine:
         deadline = time.monotonic() + TUNE_BUDGET_S
         kind = self.decode_graph
         if kind == "auto":
-            kind = ("fused" if B <= (ROWS_MAX if rows_served(cfg) else FUSED_MAX_B)
-                    else "hipblaslt")
+            kind = auto_graph(cfg, B)
         elif kind == "timed" and B > FUSED_MAX_TIMED:
             kind = "hipblaslt"
         self.step_times = {}

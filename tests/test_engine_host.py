@@ -5,7 +5,10 @@ latest earlier occurrence of the last 3, else 2, else 1 tokens proposes what
 followed it, a continuation that reaches the end reads the draft itself, and no
 occurrence repeats the last token."""
 
+import pytest
+
 from kernel_optim_amd.engine import NgramIndex, accept, draft_len
+from kernel_optim_amd.model import Qwen3Config
 
 
 def test_draft_follows_latest_trigram():
@@ -52,6 +55,19 @@ def test_accept_prefix_and_next_token():
 
 def test_draft_len_by_batch():
     assert [draft_len(b) for b in (1, 4, 5, 16, 17, 32, 33)] == [6, 6, 4, 4, 2, 2, 0]
+
+
+@pytest.mark.parametrize("tune", [True, False])
+def test_auto_takes_the_fused_graph_where_its_gemvs_read_the_weights_once(monkeypatch, tune):
+    """Up to 32 sequences at any width; up to 64 where layout 5 serves the widths, which is
+    not taken with tuning off."""
+    from kernel_optim_amd import engine
+    monkeypatch.setattr(engine, "TUNE", tune)
+    small = Qwen3Config(layers=2, vocab=64, hidden=512, inter=1024, nq=8, nkv=2)
+    assert engine.rows_served(Qwen3Config()) and not engine.rows_served(small)
+    for cfg, most in ((Qwen3Config(), 64 if tune else 32), (small, 32)):
+        for B in (1, 32, 33, 64, 65):
+            assert engine.auto_graph(cfg, B) == ("fused" if B <= most else "hipblaslt")
 
 
 def test_attention_units_per_sequence_fill_the_cus():
