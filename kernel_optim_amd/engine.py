@@ -39,6 +39,7 @@ break-even, decoding finishes on the pipelined one-token graph
 import os
 import sys
 import time
+import weakref
 
 import torch
 
@@ -83,6 +84,7 @@ WINDOW = 8               # verify steps between two acceptance checks
 HOST_MS = 0.2            # host time per verify step (wait, draft, copies)
 MIN_ADVANCE = (float(os.environ["ENGINE_MIN_ADVANCE"]) if "ENGINE_MIN_ADVANCE" in os.environ
                else None)
+PIN_RESULTS = 64 << 20   # bytes of verify results in pinned memory that callers may hold
 FUSED_VERIFY_ROWS = 16   # verify rows the fused GEMVs take in one weight pass
 
 
@@ -298,6 +300,28 @@ def decode_layer(gv, W, i, lw, attn, h, qkv, attn_out, act, k_cache, v_cache, co
     gv["down"](act, W["down"][i], h=h, nxt=_chain(gv, "down", "qkv", next_norm)[0])
 
 
+class HostCopies:
+    """Copies of device tensors on the host, a caller's to keep. They are pinned (2 MB of
+    logits arrive in 50 us, against 190-480 us through a pageable tensor) while the pinned
+    ones that callers still hold, whole or by a view, stay within ``limit`` bytes, and
+    ordinary tensors beyond: what a caller gathers is not page-locked memory."""
+
+    def __init__(self, limit, empty=torch.empty):
+        self.limit, self.empty = limit, empty
+        self.held = []   # (weak reference to the storage, bytes) of the pinned copies
+
+    def __call__(self, tensors):
+        """The copies, complete once the stream is synchronised."""
+        self.held = [(r, n) for r, n in self.held if r() is not None]
+        sizes = [t.numel() * t.element_size() for t in tensors]
+        pin = sum(n for _, n in self.held) + sum(sizes) <= self.limit
+        out = [self.empty(t.shape, dtype=t.dtype, pin_memory=pin).copy_(t, non_blocking=pin)
+               for t in tensors]
+        if pin:
+            self.held += [(weakref.ref(t.untyped_storage()), n) for t, n in zip(out, sizes)]
+        return out
+
+
 class Engine:
     def __init__(self, model_path: str, keep_logits: bool = False, spec=None,
                  decode_graph=None) -> None:
@@ -352,6 +376,7 @@ class Engine:
         self._shape = None
         self.g1 = None
         self._tile_cache = {}
+        self._results = HostCopies(PIN_RESULTS)
         # polls of a done flag before an attention + o projection wait gives up
         # (-1: the library's bound; 0: at once, which tests of that path use);
         # taken at the next setup
@@ -658,9 +683,8 @@ class Engine:
         """Replay the verify graph for rows [B, K+1] (int64: the last accepted token
         and K drafts) at positions pos [B] (of rows[:, 0]); returns the greedy ids
         [B, K+1] and, with keep_logits, the bf16 logits [B*(K+1), V], on the CPU
-        (in pinned memory: 2 MB of logits arrive in 50 us, against 190-480 us through
-        a pageable tensor). Writes K/V cache slots pos .. pos+K. Needs a setup with
-        speculation."""
+        (HostCopies: new tensors of the caller's, pinned while it holds few). Writes K/V
+        cache slots pos .. pos+K. Needs a setup with speculation."""
         if self.gk is None:
             raise ValueError("verify_step needs an engine set up with speculation (spec=True, "
                              "max_new_tokens > 2, a batch of at most 32)")
@@ -670,8 +694,7 @@ class Engine:
         self.vin.copy_(self.pin_vin, non_blocking=True)
         self._set_pos(self.pin_pos)
         self.gk.replay()
-        out = [torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t, non_blocking=True)
-               for t in ((self.vout, self.logitsT) if self.keep_logits else (self.vout,))]
+        out = self._results((self.vout, self.logitsT) if self.keep_logits else (self.vout,))
         torch.cuda.synchronize()
         return out[0], (out[1] if self.keep_logits else None)
 

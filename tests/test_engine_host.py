@@ -6,8 +6,9 @@ followed it, a continuation that reaches the end reads the draft itself, and no
 occurrence repeats the last token."""
 
 import pytest
+import torch
 
-from kernel_optim_amd.engine import NgramIndex, accept, draft_len
+from kernel_optim_amd.engine import HostCopies, NgramIndex, accept, draft_len
 from kernel_optim_amd.model import Qwen3Config
 
 
@@ -82,3 +83,30 @@ def test_attention_units_per_sequence_fill_the_cus():
         for B in range(3, 65):
             u = attn_units_per_seq(B, nkv)
             assert u >= 1 and B * nkv * u <= 1024
+
+
+@torch.inference_mode()
+def test_host_copies_are_pinned_while_few_are_held():
+    pins = []
+
+    def empty(*a, pin_memory, **kw):
+        pins.append(pin_memory)
+        return torch.empty(*a, **kw)
+
+    copies = HostCopies(4000, empty)
+    ids, logits = torch.arange(10), torch.randn(10, 90).bfloat16()   # 80 + 1800 bytes
+    for _ in range(5):   # dropped at once: the next call may pin again
+        got = copies((ids, logits))
+        assert torch.equal(got[0], ids) and torch.equal(got[1], logits)
+        del got
+    assert pins == [True] * 10
+    kept = []
+    for i in range(4):
+        kept.append([t[1:3] for t in copies((ids, logits))])   # views hold the whole
+    assert pins[10:] == [True] * 4 + [False] * 4
+    assert all(torch.equal(a, ids[1:3]) and torch.equal(b, logits[1:3]) for a, b in kept)
+    del kept[0]
+    copies((ids, logits))
+    assert pins[18:] == [True] * 2
+    huge = torch.zeros(4001, dtype=torch.uint8)
+    assert torch.equal(copies((huge,))[0], huge) and pins[-1] is False

@@ -64,6 +64,22 @@ def test_verify_step_matches_teacher_forced_oracle(dev, which, B):
     assert torch.all(best - chosen <= 2 * err + 1e-6)
 
 
+def test_held_verify_results_leave_pinned_memory_bounded(dev):
+    cfg = SMALL
+    eng = _engine(cfg, perturbed_weights(cfg, seed=17), keep_logits=True)
+    prompt = torch.randint(0, cfg.vocab, (2, 20), generator=torch.Generator().manual_seed(18))
+    list(eng.generate(prompt.tolist(), 6))
+    rows, at = torch.arange(2 * eng.T).view(2, eng.T), torch.tensor([20, 20], dtype=torch.int32)
+    size = 2 * eng.T * (8 + 2 * cfg.vocab)
+    eng._results.limit = 2 * size
+    kept = [eng.verify_step(rows, at) for _ in range(5)]
+    assert [[t.is_pinned() for t in k] for k in kept] == [[True] * 2] * 2 + [[False] * 2] * 3
+    for ids, logits in kept[1:]:
+        assert torch.equal(ids, kept[0][0]) and torch.equal(logits, kept[0][1])
+    del kept[0]
+    assert eng.verify_step(rows, at)[1].is_pinned()
+
+
 @pytest.mark.parametrize("B,min_advance,graph", [(1, 0.0, "auto"), (2, 0.0, "auto"),
                                                  (3, 0.0, "auto"), (2, 1e9, "auto"),
                                                  (2, 1e9, "hipblaslt")])
