@@ -179,7 +179,7 @@ def bench_decode(args, eng=None, B=1):
         "graph_ms_at_setup": eng.step_times,
     }
     if eng.step_kind == "fused":
-        res["gemv_cfg"] = {k: [list(g.cfg), round(g.us, 2)] for k, g in eng.gv.items()}
+        res["gemv_cfg"] = gemv_cfgs(eng.gv)
     if not args.no_cpu:
         hf = hf_cpu_model(args, eng)
         if hf is not None:
@@ -566,6 +566,12 @@ def cpu_decode_baseline_port(eng, w, seconds):
             "kind": "port",
             "sample": f"oracle.qwen3.Qwen3Oracle (bf16 F.linear, fp32 attention) on the CPU, same "
                       f"36-layer weights, B=1, 16-token prompt, {n} decode steps in {el:.1f} s"}
+
+
+def gemv_cfgs(gv):
+    """Each projection's launch configuration with the tuner's time, None where the
+    configuration was taken by rule (NaN is no JSON)."""
+    return {k: [list(g.cfg), round(g.us, 2) if g.us == g.us else None] for k, g in gv.items()}
 
 
 def bench_attention(args):

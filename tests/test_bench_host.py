@@ -3,6 +3,7 @@
 cached greedy tokens pass with full agreement, and a token planted off the argmax by
 more than the tie margin is counted and fails the check."""
 
+import json
 import os
 import sys
 
@@ -47,3 +48,17 @@ def test_teacher_forced_quality_check():
     q = bench.hf_teacher_forced_quality(m, prompt, bad, [1])
     assert not q["pass"] and q["positions_over_margin"] >= 1
     assert q["max_gap_to_argmax_logits"] > q["tie_margin_logits"]
+
+
+def test_gemv_configurations_taken_by_rule_are_valid_json():
+    import bench
+    from kernel_optim_amd.kernels.gemv import EPI_BF16, Gemv
+    tuned, ruled = (Gemv(17, 6144, 2560, EPI_BF16, norm=True) for _ in range(2))
+    tuned.us = 12.345
+    line = json.dumps(bench.gemv_cfgs(dict(a=tuned, b=ruled)))
+
+    def no_constant(name):
+        raise AssertionError(f"{name} is no JSON")
+    got = json.loads(line, parse_constant=no_constant)
+    assert got["a"][1] == round(12.345, 2)
+    assert got["b"] == [list(ruled.cfg), None]
