@@ -198,9 +198,10 @@ __device__ __forceinline__ uint32_t silu2(uint32_t g, uint32_t u) {
   const uint32_t t = pack_bf16x2(g0 / (1.0f + expf(-g0)), g1 / (1.0f + expf(-g1)));
   return pack_bf16x2(bf16lo(t) * bf16lo(u), bf16hi(t) * bf16hi(u));
 }
-__global__ __launch_bounds__(256) void silu_mul2_kernel(const uint16_t* __restrict__ gate,
+// out may be gate (each thread reads its chunk before it writes it): no __restrict__ there.
+__global__ __launch_bounds__(256) void silu_mul2_kernel(const uint16_t* gate,
                                                         const uint16_t* __restrict__ up,
-                                                        uint16_t* __restrict__ out, long long nc) {
+                                                        uint16_t* out, long long nc) {
   const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
   if (c >= nc) return;
   const uint4 g = ldg16(gate + 8 * c), u = ldg16(up + 8 * c);

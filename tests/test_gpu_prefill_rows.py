@@ -72,10 +72,11 @@ def test_silu_mul2_every_gate(dev):
         out = torch.empty_like(gate)
         silu_mul2(gate, up, out)
         assert _same(out, want)
-    short = gate[:2056].clone()          # one 8-value chunk past a workgroup; in place
-    want = F.silu(short) * short
-    silu_mul2(short, short.clone(), short)
-    assert _same(short, want)
+    for n in (8, 2056, 65536):           # in place: one chunk, one past a workgroup, all
+        short, up = gate[:n].clone(), gate.flip(0)[:n].contiguous()
+        want = F.silu(short) * up
+        silu_mul2(short, up, short)
+        assert _same(short, want)
 
 
 @pytest.mark.parametrize("B,S,kw", [(1, 8, {}), (2, 77, {}), (1, 7, {}),
