@@ -62,7 +62,8 @@ inline long long rows_scratch(int N, int tn, int slices) {
   return ROWS_XN + 2LL * ROWS_MAX * rows_parts(N, tn);
 }
 
-// Workgroups of the layout-2 grid: at most MFMA_CUS * per_cu, and of those the
+// Workgroups of the layout-2 grid: at most MFMA_CUS * per_cu (per_cu sizes the grid; with
+// one row tile a CU holds one workgroup at a time at K <= 4096, by its LDS), and of those the
 // fewest that keep the most tiles per workgroup at its minimum, so every
 // workgroup runs the same number of tiles (but the last ones, one fewer). A
 // part-filled last round leaves the busy workgroups as long as the full ones

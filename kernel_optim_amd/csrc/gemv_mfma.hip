@@ -44,7 +44,10 @@ __global__ __launch_bounds__(64 * WPG) void gemv_mfma_kernel(GemvArgs a, int nti
   // 4 S 16-byte chunks, as many loads as the rows hold; read straight into that order
   // every load touches 16 rows, half a line each (and one memory channel of 16, at the o
   // projection's row length): 16 / 4 rows, o 8.46 -> 6.66 / 6.67 -> 5.87 us, qkv 9.77 ->
-  // 9.10 / 8.69 -> 8.47.
+  // 9.10 / 8.69 -> 8.47. The buffer (85 / 136 KiB at K = 2560 / 4096) leaves a CU one
+  // workgroup, as the registers of most instances do anyhow; without a norm at K = 2560,
+  // where two fitted, a grid of two per CU did not lose (16 rows of 6144: 10.6 -> 9.0 us,
+  // one per CU 8.6 -> 7.5).
   constexpr bool XL = MT == 1 && S <= 16;
   constexpr int CPR = 4 * S;  // chunks of a row in a wavefront's K slice
   __shared__ uint4 s_x[XL ? WPG : 1][XL ? S * 68 : 1];

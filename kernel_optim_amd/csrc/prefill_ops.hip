@@ -134,7 +134,8 @@ __global__ __launch_bounds__(256) void prefill_norm_kernel(uint16_t* __restrict_
 // A head takes 32 lanes (lane r of the half: elements 4r .. 4r + 3), so a
 // wavefront works on two heads at a time, HT pairs of one token with their loads
 // issued together; the rotate_half partner (element +- 64) is 16 lanes away.
-// Grid: (tasks of 2 * HT heads, tokens / 4): cos and sin are read once per task.
+// One wavefront per item = token * tasks + task (a task: 2 * HT heads), 4 items a workgroup:
+// cos and sin are read once per task.
 constexpr int PD = 128;  // head dim
 constexpr int HT = 4;    // pairs of heads per wavefront
 

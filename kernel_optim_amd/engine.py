@@ -221,7 +221,9 @@ def build_decode_gemvs(cfg, M, raw, deadline, tiled_fn=None, tune=True, log="", 
     fused in): qkv (RMSNorm prologue, bf16 out), o (+ residual), gate/up (RMSNorm
     prologue, SwiGLU), down (+ residual), LM head (RMSNorm prologue, ARGMAX).
     ``raw`` maps each name to its per-layer row-major weights; with ``tune`` each
-    Gemv is timed over them (Gemv.tune). ``tiled_fn(name, weights)`` returns the
+    Gemv is timed over them until the deadline (Gemv.tune), or from 17 rows on, where
+    layout 5 serves it, takes its layout by rule: nothing is timed then (``us`` stays
+    NaN), and a deadline that has passed changes nothing. ``tiled_fn(name, weights)`` returns the
     MFMA-tiled copies for a projection that has tiled candidates (None: tune
     makes them). ``chain``: the caller passes decode_layer the next layer's norm, so
     qkv's input comes normalised from the layer before. Returns (gemvs, weights in each
@@ -358,8 +360,8 @@ class Engine:
     def _init(self, cfg, w, keep_logits, spec=None, decode_graph=None):
         """spec: prompt-lookup speculation on (True) or off (False); None takes
         ENGINE_SPEC (off unless set to 1). decode_graph: "auto" (the fused-GEMV
-        decode graph up to FUSED_MAX_B sequences, the hipBLASLt graph above),
-        "timed" (capture both up to FUSED_MAX_TIMED sequences, time them at setup
+        decode graph up to 32 sequences, or 64 where auto_graph says so, the
+        hipBLASLt graph above), "timed" (capture both up to FUSED_MAX_TIMED sequences, time them at setup
         and keep the faster), "fused" or "hipblaslt"; None takes
         ENGINE_DECODE_GRAPH (auto unless set)."""
         self.spec = SPEC if spec is None else bool(spec)
@@ -457,8 +459,8 @@ class Engine:
         self._shape = key
 
     def _setup_fused(self, raw, deadline):
-        """The fused-GEMV decode step: tuned GEMVs (with MFMA weight copies where
-        the tuner takes them) and its captured graph."""
+        """The fused-GEMV decode step: its GEMVs (build_decode_gemvs, with MFMA weight
+        copies where their layouts read them) and its captured graph."""
         self.gv, self.gw = build_decode_gemvs(self.cfg, self.B, raw, deadline, self._tiled,
                                               tune=TUNE, chain=True)
         return self._capture(self._step1)

@@ -131,7 +131,7 @@ class Gemv:
         Layout 1 (a wavefront per row group) is the batch-1..4 path; layout 0
         serves every batch up to 16 rows per launch with VALU dot products;
         layout 2 puts 2..16 rows on MFMA (``(2, per_cu, 0)``: a persistent grid
-        of at most 256 x per_cu workgroups, the fewest that keep the most tiles
+        of at most 256 x per_cu workgroups (resident one per CU up to K = 4096), the fewest that keep the most tiles
         per workgroup at its minimum; ``(2, per_cu, 2)``: 32 rows per weight
         pass, offered above 16 rows), layout 3 splits its tiles' K range and
         layout 4 (``(4, 10, 0)``; ``(4, 10, 2)`` / ``(4, 10, 4)`` with 32 / 64

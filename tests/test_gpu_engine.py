@@ -194,21 +194,23 @@ def test_hipblaslt_decode_graph_qwen3_4b_width(dev):
     assert err < LOGIT_ATOL
 
 
-@pytest.mark.parametrize("B", [32, 40])
+@pytest.mark.parametrize("B", [32, 40, 64, 65])
 def test_fused_decode_graph_above_16_rows(dev, B):
-    """The fused decode graph, forced, at 32 and 40 sequences (2-layer Qwen3-4B
-    width): the GEMVs run 32-row slices (two MFMA row tiles per weight pass, where
-    the tuner takes them) and, at 40, an 8-row slice after them. Tokens and
-    logits against the oracle's teacher-forced replay, as the B = 3 hipBLASLt
-    test."""
+    """The fused decode graph at 32, 40 and 64 sequences, auto's choice up to there, and
+    forced at 65 (2-layer Qwen3-4B width): the projections run on layout 5, up to 64 rows
+    per weight pass (at 65 a second pass of one row, unchained), the LM head at 32 on layout
+    2's two row tiles. Tokens and logits against the oracle's teacher-forced replay, as the
+    B = 3 hipBLASLt test."""
     cfg = Qwen3Config(layers=2)
     w = random_weights(cfg, seed=9)
     prompt = torch.randint(0, cfg.vocab, (B, 48), generator=torch.Generator().manual_seed(B))
     n = 8
-    eng = _engine(cfg, w, decode_graph="fused")
+    eng = _engine(cfg, w, decode_graph="auto" if B <= 64 else "fused")
     toks, logits = eng.trace(prompt.tolist(), n)
     assert eng.step_kind == "fused"
     cfgs = {k: g.cfg for k, g in eng.gv.items()}
+    assert all(cfgs[k][0] == 5 for k in ("qkv", "o", "gu", "down"))
+    assert cfgs["lm"] == ((2, 1, 2) if B == 32 else (5, 6, 1))
     del eng
     torch.cuda.empty_cache()
     replay = Qwen3Oracle(cfg, w, B=B, cap=64).teacher_forced(prompt, toks)
@@ -236,7 +238,8 @@ def test_timed_choice_keeps_the_faster_decode_graph(dev):
 
 def test_auto_builds_one_decode_graph(dev):
     """decode_graph="auto" (the default) captures only the fused-GEMV graph up to
-    FUSED_MAX_B sequences: no hipBLASLt graph is built or timed."""
+    FUSED_MAX_B sequences at widths that layout 5 does not serve: no hipBLASLt graph is
+    built or timed."""
     from kernel_optim_amd.engine import FUSED_MAX_B
     cfg = SMALL
     w = perturbed_weights(cfg, seed=11)
@@ -255,7 +258,7 @@ def test_auto_builds_one_decode_graph(dev):
 @pytest.mark.parametrize("kind", ["auto", "timed"])
 def test_batch_above_the_fused_limit_takes_hipblaslt(dev, kind):
     """Above the fused limit only the hipBLASLt graph is set up: B = FUSED_MAX_B + 1
-    (33) with auto, B = FUSED_MAX_TIMED + 1 (65) with the timed choice (the
+    (33) with auto at widths that layout 5 does not serve, B = FUSED_MAX_TIMED + 1 (65) with the timed choice (the
     reference's rule, engine.py:197-199), and every sequence's tokens and logits
     meet the oracle replay's bar."""
     from kernel_optim_amd.engine import FUSED_MAX_B, FUSED_MAX_TIMED
