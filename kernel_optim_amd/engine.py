@@ -69,9 +69,10 @@ ATTN_SPLIT = int(os.environ.get("ENGINE_ATTN_SPLIT", "-1"))
 # captures both up to FUSED_MAX_TIMED and keeps the faster, as the reference does
 # (engine.py:197-208); "fused" or "hipblaslt" takes one
 DECODE_GRAPH = os.environ.get("ENGINE_DECODE_GRAPH", "auto")
-# The fused GEMVs of any width read each weight once for up to 32 rows (B = 32: 8,619
-# tok/s against 7,544 on hipBLASLt); at 33..64 rows only layout 5 does, so "auto" takes
-# the fused step there for the widths that it serves (rows_served).
+# The fused GEMVs of any width read each weight once for up to 32 rows (layouts 2 and 4 at
+# Qwen3-4B's widths, B = 32: 8,619 tok/s against 7,544 on hipBLASLt; layout 5 10,440); at
+# 33..64 rows only layout 5 does, so "auto" takes the fused step there for the widths that
+# it serves (rows_served).
 FUSED_MAX_B = 32
 FUSED_MAX_TIMED = 64  # "timed": both graphs up to here (engine.py:44)
 # verify-step attention: the K+1 tokens of a sequence as rows of the one-token
